@@ -199,6 +199,14 @@ __device__ __forceinline__ void store_cpx(global_t<__half2>* p, long i, float2 v
     reinterpret_cast<global_t<unsigned>*>(p)[i] = lo | (hi << 16);
 }
 
+// elements 2 m and 2 m + 1 of an 8-byte aligned line of half pairs
+__device__ __forceinline__ void store_cpx_pair(global_t<__half2>* p, long m, float2 a, float2 b) {
+    typedef unsigned uvec2 __attribute__((ext_vector_type(2)));
+    const unsigned   x = (unsigned)__half_as_ushort(__float2half_rn(a.x)) | ((unsigned)__half_as_ushort(__float2half_rn(a.y)) << 16);
+    const unsigned   y = (unsigned)__half_as_ushort(__float2half_rn(b.x)) | ((unsigned)__half_as_ushort(__float2half_rn(b.y)) << 16);
+    reinterpret_cast<global_t<uvec2>*>(p)[m] = uvec2{x, y};
+}
+
 // ---------------------------------------------------------------- small DFTs in registers
 // In-place radix-R DFT (R = 2,4,8,16) by compile-time radix-2 decimation in time.
 // Constant twiddles W_R^k are exact decimal expansions; multiplications by 1 and

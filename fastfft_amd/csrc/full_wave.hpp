@@ -1,13 +1,17 @@
-// Full-length forward line transforms (no size change) with one workgroup of
-// Q wavefronts per line: the R2C x-pass and the C2C y-pass of an unpadded
-// FwdFFT (the reference's block_fft_kernel_R2C_NONE_XY and C2C_NONE,
-// src/fastfft/FastFFT.cu:1055-1077, :1348-1367), used for the micrograph
-// spectrum of the correlation path.
+// Forward line transforms of any non-zero length L <= N with one workgroup of Q
+// wavefronts per line: the C2C y-pass of a FwdFFT, padded or not, and the R2C x-pass
+// of rows too short for the pair kernel (the reference's block_fft_kernel_R2C_NONE_XY,
+// R2C_INCREASE_XY, C2C_NONE and C2C_INCREASE, src/fastfft/FastFFT.cu:1055-1166,
+// :1348-1367).
 //
 // N = P*Q is split decimation-in-frequency style:
 //   y_q[m]      = sum_s x[s P + m] W_Q^{s q}          (radix-Q pass over the line in LDS)
 //   X[Q k' + q] = FFT_P( y_q[m] W_N^{m q} )[k']         (wave q, register Stockham)
-// The line is read with coalesced loads into LDS.  A unit-stride output line is
+// The line is read with coalesced loads into LDS, zeros from L on: a padded line costs
+// the arithmetic of a whole one but reads L values only, and the stores of the N outputs
+// bound it.  The generic line kernel, which runs one P-point transform per output residue
+// (P >= L) in turn, took 17.3 us for 257 lines of 64 in 512 points and 79 us for 2049 of
+// 2750 in 4096 (here about 4 and 21 us).  A unit-stride output line is
 // written through LDS with 16-byte stores; a strided one (the transposed x-pass
 // output) one value per output line, with each XCD owning a contiguous range
 // of lines so that the partial lines meet in one L2.
@@ -17,9 +21,9 @@
 
 namespace fastfft_amd {
 
-template <int P, int Q, typename TIn, bool REAL>
+template <int P, int Q, typename TIn, bool REAL, typename TOut>
 __global__ void __launch_bounds__(64 * Q)
-        k_fwd_full_wave(const TIn* __restrict__ in, LineMap im, float2* __restrict__ out, LineMap om, int nout, int nlines,
+        k_fwd_full_wave(const TIn* __restrict__ in, LineMap im, int L, TOut* __restrict__ out, LineMap om, int nout, int nlines,
                         float pre_scale, const float2* __restrict__ tw) {
     constexpr int T = 64, E = P / T, N = P * Q, NT = T * Q;
     using FFT       = WaveFFT<P>;
@@ -43,10 +47,13 @@ __global__ void __launch_bounds__(64 * Q)
 #pragma unroll
         for ( int r = 0; r < N / NT; r++ ) {
             const int n = threadIdx.x + NT * r;
-            if constexpr ( REAL )
-                z[r] = make_float2(load_real(lp, n * im.es), 0.f);
-            else
-                z[r] = load_cpx(lp, n * im.es);
+            z[r]        = make_float2(0.f, 0.f);
+            if ( n < L ) {
+                if constexpr ( REAL )
+                    z[r].x = load_real(lp, n * im.es);
+                else
+                    z[r] = load_cpx(lp, n * im.es);
+            }
         }
         tws.store(s_twp, s_twn);
 #pragma unroll
@@ -84,9 +91,9 @@ __global__ void __launch_bounds__(64 * Q)
         v[i] = cmul(cmul(lds[q * P + t + T * i], twm[N + ((T * i * q) & (N - 1))]), lw);
     __syncthreads( );
     fft.template run<-1>(v, lds + q * FFT::SLOTS, t);
-    float2* op = out + om.base(line);
+    auto* op = as_global(out) + om.base(line);
     if ( om.es == 1 ) {
-        // natural order through LDS, then 16-byte stores (op is 16-byte aligned)
+        // natural order through LDS, then pair stores (op aligned to two values)
         __syncthreads( );
 #pragma unroll
         for ( int i = 0; i < E; i++ )
@@ -95,11 +102,11 @@ __global__ void __launch_bounds__(64 * Q)
         for ( int m = threadIdx.x; 2 * m < nout; m += NT ) {
             const float2 u0 = lds[dec_slot<P, Q>(2 * m)];
             if ( 2 * m + 1 < nout ) {
-                const float2 u1                  = lds[dec_slot<P, Q>(2 * m + 1)];
-                reinterpret_cast<float4*>(op)[m] = make_float4(u0.x, u0.y, u1.x, u1.y);
+                const float2 u1 = lds[dec_slot<P, Q>(2 * m + 1)];
+                store_cpx_pair(op, m, u0, u1);
             }
             else {
-                op[2 * m] = u0;
+                store_cpx(op, 2 * m, u0);
             }
         }
     }
@@ -108,7 +115,7 @@ __global__ void __launch_bounds__(64 * Q)
         for ( int i = 0; i < E; i++ ) {
             const int k = Q * (t + T * i) + q;
             if ( k < nout )
-                op[k * om.es] = v[i];
+                store_cpx(op, k * om.es, v[i]);
         }
     }
 }

@@ -180,32 +180,29 @@ static hipError_t try_r2c_wave(const Stage& s, const StageIO& io, const float2* 
     return hipErrorNotSupported;
 }
 
-// Full-length lines (L = N, 256 <= N <= 8192) with a float2 output: one
-// workgroup per line, P = 512 (256 for N = 256) and Q = N / P.
+// Lines of 256 <= N <= 8192 points with L <= N non-zero inputs: one workgroup per
+// line, P = 512 (256 for N = 256) and Q = N / P.
+template <int P, int Q, typename TIn, bool REAL, typename TOut>
+static hipError_t go_full_wave_t(const Stage& s, const StageIO& io, const float2* tw, hipStream_t st) {
+    launch_kernel<k_fwd_full_wave<P, Q, TIn, REAL, TOut>>(dim3((unsigned)s.nlines), dim3(64 * Q), 0, st,
+            static_cast<const TIn*>(io.src), to_device(s.im), s.L, static_cast<TOut*>(io.dst), to_device(s.om), s.nout,
+            s.nlines, io.scale, tw);
+    return hipGetLastError( );
+}
+
 template <int P, int Q>
 static hipError_t go_full_wave(const Stage& s, const StageIO& io, const float2* tw, hipStream_t st) {
-    const dim3 grid((unsigned)s.nlines), block(64 * Q);
     if ( io.src_real ) {
-        if ( io.src_rt == RealT::f32 )
-            launch_kernel<k_fwd_full_wave<P, Q, float, true>>(grid, block, 0, st, static_cast<const float*>(io.src), to_device(s.im),
-                                                                       static_cast<float2*>(io.dst), to_device(s.om),
-                                                                       s.nout, s.nlines, io.scale, tw);
-        else
-            launch_kernel<k_fwd_full_wave<P, Q, __half, true>>(grid, block, 0, st, static_cast<const __half*>(io.src), to_device(s.im),
-                                                                        static_cast<float2*>(io.dst), to_device(s.om),
-                                                                        s.nout, s.nlines, io.scale, tw);
+        if ( io.dst_ct != CpxT::c64 )
+            return hipErrorNotSupported;
+        return io.src_rt == RealT::f32 ? go_full_wave_t<P, Q, float, true, float2>(s, io, tw, st)
+                                       : go_full_wave_t<P, Q, __half, true, float2>(s, io, tw, st);
     }
-    else {
-        if ( io.src_ct == CpxT::c64 )
-            launch_kernel<k_fwd_full_wave<P, Q, float2, false>>(grid, block, 0, st, static_cast<const float2*>(io.src), to_device(s.im),
-                                                                         static_cast<float2*>(io.dst), to_device(s.om),
-                                                                         s.nout, s.nlines, io.scale, tw);
-        else
-            launch_kernel<k_fwd_full_wave<P, Q, __half2, false>>(grid, block, 0, st, static_cast<const __half2*>(io.src),
-                                                                          to_device(s.im), static_cast<float2*>(io.dst),
-                                                                          to_device(s.om), s.nout, s.nlines, io.scale, tw);
-    }
-    return hipGetLastError( );
+    // (the planner's complex forward stages read FP32 intermediates)
+    if ( io.src_ct != CpxT::c64 )
+        return hipErrorNotSupported;
+    return io.dst_ct == CpxT::c64 ? go_full_wave_t<P, Q, float2, false, float2>(s, io, tw, st)
+                                  : go_full_wave_t<P, Q, float2, false, __half2>(s, io, tw, st);
 }
 
 // Full-length real lines into a transposed spectrum (lines adjacent, even element
@@ -242,9 +239,9 @@ static bool full_wave_pair_covers(const Stage& s, const StageIO& io) {
 }
 
 static hipError_t try_full_wave(const Stage& s, const StageIO& io, const float2* tw, hipStream_t st) {
-    if ( s.L != s.N || io.dst_real || io.dst_ct != CpxT::c64 || s.nout > s.N )
+    if ( s.L > s.N || io.dst_real || s.nout > s.N )
         return hipErrorNotSupported;
-    if ( full_wave_pair_covers(s, io) ) {
+    if ( s.L == s.N && io.dst_ct == CpxT::c64 && full_wave_pair_covers(s, io) ) {
         switch ( s.N ) {
             case 1024: return go_full_wave_pair<512, 2>(s, io, tw, st);
             case 2048: return go_full_wave_pair<512, 4>(s, io, tw, st);
@@ -269,15 +266,17 @@ static hipError_t try_full_wave(const Stage& s, const StageIO& io, const float2*
 }
 
 hipError_t launch_fwd(const Stage& s, const StageIO& io, const float2* tw, hipStream_t st) {
-    // a unit-stride output row is written with 16-byte stores: even line offsets, aligned base
-    const bool rows_ok = s.om.es != 1 || (s.om.s1 % 2 == 0 && s.om.s2 % 2 == 0 &&
-                                          reinterpret_cast<std::uintptr_t>(io.dst) % 16 == 0);
+    // a unit-stride output row is written two values at a time: even line offsets, aligned base
+    const std::uintptr_t pair_bytes = io.dst_ct == CpxT::c64 ? 16 : 8;
+    const bool           rows_ok    = s.om.es != 1 || (s.om.s1 % 2 == 0 && s.om.s2 % 2 == 0 &&
+                                          reinterpret_cast<std::uintptr_t>(io.dst) % pair_bytes == 0);
+    const bool           full_lines = rows_ok && ! env_int("FASTFFT_NO_WAVE_ROWS", 0) && ! env_int("FASTFFT_NO_FULL_LINES", 0);
     if ( io.src_real && ! io.dst_real && io.dst_ct == CpxT::c64 && ! env_int("FASTFFT_NO_WAVE_ROWS", 0) ) {
         hipError_t e = launch_r2c_packed(s, io.src, io.dst, io.src_rt, s.nlines, io.scale, tw, nullptr, 1, st);
         if ( e != hipErrorNotSupported )
             return e;
     }
-    if ( rows_ok && ! env_int("FASTFFT_NO_WAVE_ROWS", 0) && ! env_int("FASTFFT_NO_FULL_LINES", 0) ) {
+    if ( full_lines && s.L == s.N ) {
         hipError_t e = try_full_wave(s, io, tw, st);
         if ( e != hipErrorNotSupported )
             return e;
@@ -287,6 +286,13 @@ hipError_t launch_fwd(const Stage& s, const StageIO& io, const float2* tw, hipSt
     if ( (s.kind == StageKind::fwd_cpx || (s.kind == StageKind::fwd_real && s.om.es != 1)) &&
          ! env_int("FASTFFT_NO_WAVE_ROWS", 0) ) {
         hipError_t e = launch_tile_lines(s, io, tw, st);
+        if ( e != hipErrorNotSupported )
+            return e;
+    }
+    // padded lines the tiles leave: unit-stride complex lines, and real rows into a transposed
+    // spectrum that no sub-transform kernel takes
+    if ( full_lines && s.L < s.N && (io.src_real ? s.om.es != 1 && ! r2c_rows_shape(s) : s.im.es == 1 && s.om.es == 1) ) {
+        hipError_t e = try_full_wave(s, io, tw, st);
         if ( e != hipErrorNotSupported )
             return e;
     }
