@@ -26,7 +26,8 @@ COMMON = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
 SOURCES = ["planner.cpp", "capi.cpp", "launch_fwd.hip", "launch_inv.hip", "launch_xcorr.hip", "launch_tile.hip", "misc.hip", "scratch.hip",
            "tuning.cpp"]
 HEADERS = ["fft_core.hpp", "line_kernels.hpp", "launch.hpp", "launch_common.hpp", "plan.hpp", "wave_fft.hpp",
-           "xcorr_col.hpp", "rows_wave.hpp", "items.hpp", "full_wave.hpp", "window_rows.hpp", "xcorr_toeplitz.hpp", "tile_lines.hpp", "rows_packed.hpp", "tuning.hpp"]
+           "xcorr_col.hpp", "rows_wave.hpp", "items.hpp", "full_wave.hpp", "window_rows.hpp", "xcorr_toeplitz.hpp", "tile_lines.hpp", "rows_packed.hpp",
+           "pair_rows.hpp", "tuning.hpp"]
 
 
 def _needs(obj: str, src: str) -> bool:

@@ -331,6 +331,7 @@ static fastfft_status ensure_device_state(fastfft_plan p, float2** tw) {
             p->ws = nullptr;
         }
         workspace_elems(p->st, p->ws_a, p->ws_b);
+        p->ws_a      = (p->ws_a + 15) / 16 * 16; // ws_b starts 128-byte aligned
         size_t bytes = sizeof(float2) * (p->ws_a + p->ws_b);
         if ( bytes < 256 )
             bytes = 256;

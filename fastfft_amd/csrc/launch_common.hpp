@@ -60,6 +60,41 @@ hipError_t prepare_launch(K kernel, int nlines, dim3& grid, dim3& block, size_t&
 
 inline int twiddle_stride(int N) { return kTwiddleN / N; }
 
+// Integer value of a tuning environment variable (dflt when unset).  Read on
+// every call so that tests can switch kernels within one process; getenv is
+// cheap next to a kernel launch.
+inline int env_int(const char* name, int dflt) {
+    const char* v = std::getenv(name);
+    return (v && v[0]) ? std::atoi(v) : dflt;
+}
+
+// Calls f(N, PPW) for the pair-row kernels (pair_rows.hpp): rows of N points, PPW pairs per
+// workgroup, at most FASTFFT_PAIR_GROUP.  Four pairs make 64-byte segments (workgroups of 1024
+// threads at N = 4096; 8192-point rows fit two): 4096^2 forward 71 us with one pair, 56 with
+// two, 56-57 with four; 2730 rows of 4096 points 65, 50 and 45.  Below 64 workgroups' worth of
+// pairs the group is halved to keep CUs busy: 255 rows of 2048 points 16.4, 16.8 and 18.2 us.
+template <class F>
+hipError_t pair_rows_dispatch(int N, int nrows, F&& f) {
+    const int npairs = (nrows + 1) / 2, cap = env_int("FASTFFT_PAIR_GROUP", 4);
+    int       g      = N == 8192 ? 2 : 4;
+    while ( g > 1 && (g > cap || npairs < 64 * g) )
+        g /= 2;
+    auto by_n = [&](auto nc) -> hipError_t {
+        constexpr int NN = decltype(nc)::value;
+        if constexpr ( NN <= 4096 )
+            if ( g == 4 )
+                return f(nc, std::integral_constant<int, 4>{ });
+        return g >= 2 ? f(nc, std::integral_constant<int, 2>{ }) : f(nc, std::integral_constant<int, 1>{ });
+    };
+    switch ( N ) {
+        case 1024: return by_n(std::integral_constant<int, 1024>{ });
+        case 2048: return by_n(std::integral_constant<int, 2048>{ });
+        case 4096: return by_n(std::integral_constant<int, 4096>{ });
+        case 8192: return by_n(std::integral_constant<int, 8192>{ });
+        default: return hipErrorNotSupported;
+    }
+}
+
 // A type whose mangled name spells out the kernel K with its template arguments.
 template <auto K>
 struct KernelTag { };
@@ -70,14 +105,6 @@ inline void launch_kernel(dim3 grid, dim3 block, size_t lds, hipStream_t st, A&&
     if ( log_enabled( ) )
         log_launch(typeid(KernelTag<K>).name( ), grid, block, lds);
     K<<<grid, block, lds, st>>>(std::forward<A>(a)...);
-}
-
-// Integer value of a tuning environment variable (dflt when unset).  Read on
-// every call so that tests can switch kernels within one process; getenv is
-// cheap next to a kernel launch.
-inline int env_int(const char* name, int dflt) {
-    const char* v = std::getenv(name);
-    return (v && v[0]) ? std::atoi(v) : dflt;
 }
 
 } // namespace fastfft_amd

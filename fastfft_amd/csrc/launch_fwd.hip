@@ -3,6 +3,7 @@
 
 #include "full_wave.hpp"
 #include "launch_common.hpp"
+#include "pair_rows.hpp"
 #include "rows_packed.hpp"
 #include "rows_wave.hpp"
 
@@ -205,55 +206,34 @@ static hipError_t go_full_wave(const Stage& s, const StageIO& io, const float2* 
                                   : go_full_wave_t<P, Q, float2, false, __half2>(s, io, tw, st);
 }
 
-// Full-length real lines into a transposed spectrum (lines adjacent, even element
-// step, 16-byte aligned output): two lines per workgroup as one complex line.
-// PPW pairs per workgroup (FASTFFT_PAIR_GROUP = 1, 2 or 4 caps it; by default 4 for
-// 4096-point rows, 2 for the other lengths where the pair count allows and a workgroup
-// of 2 Q waves fits).
-template <int P, int Q, int PPW>
-static hipError_t go_full_wave_pair_g(const Stage& s, const StageIO& io, const float2* tw, hipStream_t st) {
-    const int  npairs = s.nlines / 2;
-    const dim3 grid((unsigned)(npairs / PPW)), block(64 * Q * PPW);
+// Real rows of 1024 .. 8192 points into a transposed spectrum, two rows as one complex
+// line (pair_rows.hpp), PPW pairs per workgroup.
+template <int N, int PPW>
+static hipError_t go_pair_rows(const Stage& s, const StageIO& io, const float2* tw, hipStream_t st) {
+    const dim3 grid((unsigned)(((s.nlines + 1) / 2 + PPW - 1) / PPW)), block(N / kPairE * PPW);
     if ( io.src_rt == RealT::f32 )
-        launch_kernel<k_fwd_full_wave_pair<P, Q, float, PPW>>(grid, block, 0, st, static_cast<const float*>(io.src),
-                to_device(s.im), static_cast<float2*>(io.dst), to_device(s.om), s.nout, npairs, io.scale, tw);
+        launch_kernel<k_r2c_pair_rows<N, PPW, float>>(grid, block, 0, st, static_cast<const float*>(io.src), to_device(s.im),
+                s.L, static_cast<float2*>(io.dst), to_device(s.om), s.nout, s.nlines, io.scale, tw);
     else
-        launch_kernel<k_fwd_full_wave_pair<P, Q, __half, PPW>>(grid, block, 0, st, static_cast<const __half*>(io.src),
-                to_device(s.im), static_cast<float2*>(io.dst), to_device(s.om), s.nout, npairs, io.scale, tw);
+        launch_kernel<k_r2c_pair_rows<N, PPW, __half>>(grid, block, 0, st, static_cast<const __half*>(io.src),
+                to_device(s.im), s.L, static_cast<float2*>(io.dst), to_device(s.om), s.nout, s.nlines, io.scale, tw);
     return hipGetLastError( );
 }
 
-template <int P, int Q>
-static hipError_t go_full_wave_pair(const Stage& s, const StageIO& io, const float2* tw, hipStream_t st) {
-    if constexpr ( Q <= 8 ) {
-        if ( env_int("FASTFFT_PAIR_GROUP", 4) >= 2 && (s.nlines / 2) % 2 == 0 )
-            return go_full_wave_pair_g<P, Q, 2>(s, io, tw, st);
-    }
-    return go_full_wave_pair_g<P, Q, 1>(s, io, tw, st);
-}
-
-static bool full_wave_pair_covers(const Stage& s, const StageIO& io) {
-    return io.src_real && s.nlines >= 2 && s.nlines % 2 == 0 && s.om.n2 == 1 && s.om.s1 == 1 && s.om.es % 2 == 0 &&
-           s.im.n2 == 1 && reinterpret_cast<std::uintptr_t>(io.dst) % 16 == 0 && s.N >= 1024 &&
-           ! env_int("FASTFFT_NO_PAIR_LINES", 0);
+static hipError_t try_pair_rows(const Stage& s, const StageIO& io, const float2* tw, hipStream_t st) {
+    if ( s.kind != StageKind::fwd_real || ! io.src_real || io.dst_real || io.dst_ct != CpxT::c64 || s.nlines < 1 ||
+         s.L > s.N || s.nout < 1 || s.nout > s.N / 2 + 1 || s.im.n2 != 1 || s.im.es != 1 || s.om.n2 != 1 || s.om.s1 != 1 ||
+         s.om.es % 2 != 0 || s.om.es < s.nlines ||
+         reinterpret_cast<std::uintptr_t>(io.dst) % 16 != 0 || env_int("FASTFFT_NO_PAIR_LINES", 0) )
+        return hipErrorNotSupported;
+    return pair_rows_dispatch(s.N, s.nlines, [&](auto nc, auto gc) {
+        return go_pair_rows<decltype(nc)::value, decltype(gc)::value>(s, io, tw, st);
+    });
 }
 
 static hipError_t try_full_wave(const Stage& s, const StageIO& io, const float2* tw, hipStream_t st) {
     if ( s.L > s.N || io.dst_real || s.nout > s.N )
         return hipErrorNotSupported;
-    if ( s.L == s.N && io.dst_ct == CpxT::c64 && full_wave_pair_covers(s, io) ) {
-        switch ( s.N ) {
-            case 1024: return go_full_wave_pair<512, 2>(s, io, tw, st);
-            case 2048: return go_full_wave_pair<512, 4>(s, io, tw, st);
-            case 4096:
-                // four pairs of 4096-point rows per workgroup on 1024-point sub-transforms (Q = 4)
-                if ( env_int("FASTFFT_PAIR_GROUP", 4) >= 4 && (s.nlines / 2) % 4 == 0 )
-                    return go_full_wave_pair_g<1024, 4, 4>(s, io, tw, st);
-                return go_full_wave_pair<512, 8>(s, io, tw, st);
-            case 8192: return go_full_wave_pair<512, 16>(s, io, tw, st);
-            default: break;
-        }
-    }
     switch ( s.N ) {
         case 256: return go_full_wave<256, 1>(s, io, tw, st);
         case 512: return go_full_wave<512, 1>(s, io, tw, st);
@@ -271,6 +251,13 @@ hipError_t launch_fwd(const Stage& s, const StageIO& io, const float2* tw, hipSt
     const bool           rows_ok    = s.om.es != 1 || (s.om.s1 % 2 == 0 && s.om.s2 % 2 == 0 &&
                                           reinterpret_cast<std::uintptr_t>(io.dst) % pair_bytes == 0);
     const bool           full_lines = rows_ok && ! env_int("FASTFFT_NO_WAVE_ROWS", 0) && ! env_int("FASTFFT_NO_FULL_LINES", 0);
+    // real rows of 1024 points and up into a transposed spectrum (1024^2: 14.6 us with the
+    // one-wave packed rows, 13.3-13.8 here; 384^2 templates' row-major rows do not come here)
+    if ( full_lines ) {
+        hipError_t e = try_pair_rows(s, io, tw, st);
+        if ( e != hipErrorNotSupported )
+            return e;
+    }
     if ( io.src_real && ! io.dst_real && io.dst_ct == CpxT::c64 && ! env_int("FASTFFT_NO_WAVE_ROWS", 0) ) {
         hipError_t e = launch_r2c_packed(s, io.src, io.dst, io.src_rt, s.nlines, io.scale, tw, nullptr, 1, st);
         if ( e != hipErrorNotSupported )

@@ -1,6 +1,9 @@
 // Inverse line stages: C2C y/z passes (output pruned) and the C2R x-pass.
 #include "full_wave.hpp"
+#include <cstdint>
+
 #include "launch_common.hpp"
+#include "pair_rows.hpp"
 #include "rows_packed.hpp"
 #include "rows_wave.hpp"
 #include "window_rows.hpp"
@@ -482,9 +485,37 @@ static hipError_t try_window(const Stage& s, const StageIO& io, const float2* tw
     }
 }
 
+// C2R rows of 1024 .. 8192 points from a transposed spectrum, any window, two rows as one
+// complex line (pair_rows.hpp).
+template <int N, int PPW>
+static hipError_t go_c2r_pair_rows(const Stage& s, const StageIO& io, const float2* tw, hipStream_t st) {
+    const dim3 grid((unsigned)(((s.nlines + 1) / 2 + PPW - 1) / PPW)), block(N / kPairE * PPW);
+    const int  o = ((s.o % s.N) + s.N) % s.N;
+    if ( io.dst_rt == RealT::f32 )
+        launch_kernel<k_c2r_pair_rows<N, PPW, float>>(grid, block, 0, st, static_cast<const float2*>(io.src), to_device(s.im),
+                static_cast<float*>(io.dst), to_device(s.om), s.M, o, s.nlines, io.scale, tw);
+    else
+        launch_kernel<k_c2r_pair_rows<N, PPW, __half>>(grid, block, 0, st, static_cast<const float2*>(io.src),
+                to_device(s.im), static_cast<__half*>(io.dst), to_device(s.om), s.M, o, s.nlines, io.scale, tw);
+    return hipGetLastError( );
+}
+
+static hipError_t try_c2r_pair_rows(const Stage& s, const StageIO& io, const float2* tw, hipStream_t st) {
+    if ( s.kind != StageKind::inv_c2r || io.amax || io.src_real || io.src_ct != CpxT::c64 || ! io.dst_real || s.nlines < 1 ||
+         s.M < 1 || s.M > s.N || s.im.n2 != 1 || s.im.s1 != 1 || s.im.es % 2 != 0 || s.im.es < s.nlines ||
+         s.om.n2 != 1 || s.om.es != 1 || reinterpret_cast<std::uintptr_t>(io.src) % 16 != 0 ||
+         env_int("FASTFFT_NO_PAIR_LINES", 0) || env_int("FASTFFT_NO_FULL_LINES", 0) )
+        return hipErrorNotSupported;
+    return pair_rows_dispatch(s.N, s.nlines, [&](auto nc, auto gc) {
+        return go_c2r_pair_rows<decltype(nc)::value, decltype(gc)::value>(s, io, tw, st);
+    });
+}
+
 hipError_t launch_inv(const Stage& s, const StageIO& io, const float2* tw, hipStream_t st) {
     if ( ! env_int("FASTFFT_NO_WAVE_ROWS", 0) ) {
-        hipError_t e = try_c2r_packed(s, io, tw, st);
+        hipError_t e = try_c2r_pair_rows(s, io, tw, st);
+        if ( e == hipErrorNotSupported )
+            e = try_c2r_packed(s, io, tw, st);
         if ( e == hipErrorNotSupported )
             e = try_c2r_window_packed(s, io, tw, st);
         if ( e != hipErrorNotSupported )

@@ -1,0 +1,291 @@
+// Real rows of N = 1024 .. 8192 points against a transposed spectrum, two rows as one
+// complex line: the R2C x-pass of a FwdFFT (any non-zero length L <= N) and the C2R
+// x-pass of an InvFFT (any window), the reference's block_fft_kernel_R2C_NONE_XY,
+// R2C_INCREASE_XY, C2R_NONE_XY and C2R_DECREASE_XY (src/fastfft/FastFFT.cu:1055-1166,
+// :1641-1692), which transform one real row as a complex line each.
+//
+//   z = a + i b,  Z = FFT_N(z):  A[k] = (Z[k] + conj Z[N-k]) / 2,  B[k] = -i (Z[k] - conj Z[N-k]) / 2
+//   Z[k] = A[k] + i B[k],  Z[N-k] = conj A[k] + i conj B[k]:       z = IFFT_N(Z), a = Re z, b = Im z
+//
+// The spectrum is stored A[kx][y]: the 2 PPW rows of a workgroup are one 16 PPW-byte
+// segment of every kx, moved 16 bytes per lane; the rows themselves are unit stride.
+// 16 values per thread in registers (T = N / 16 threads per pair), loaded and stored
+// directly, radix-16 Stockham passes, and every exchange moves the real and then the
+// imaginary parts through one LDS buffer of N floats per pair.  That halves the LDS of a
+// pair, and immediate offsets keep the addresses out of the registers (64 at most), so two
+// workgroups of 1024 threads share a CU and one loads or stores while the other computes.
+// Bound by arithmetic and memory about alike: 4096^2 (134 MB) takes 30.7 us forward and
+// 29.7 us inverse, 4.4-4.5 TB/s, where complex exchanges with one workgroup per CU took
+// 38.6 us forward and one row per workgroup with 8-byte gathers 51.7 us inverse.
+#pragma once
+
+#include "rows_wave.hpp"
+
+namespace fastfft_amd {
+
+constexpr int kPairE = 16; // values per thread
+
+// Exchange slot of element k: one pad word per 16, so that the scatters of the radix-16
+// passes (lane strides 16 and 256) and the unit-stride gathers fall on distinct banks.
+// Slots 16 m elements apart lie 17 m words apart: one address and immediate offsets.
+__device__ __forceinline__ int pair_slot(int k) { return k + (k >> 4); }
+constexpr int                  pair_step(int k) { return k + k / 16; }
+// Floats per pair (slot N, a copy of element 0 beside the mirrored element N - k, included):
+// PPW consecutive pairs start 64 / PPW banks apart, so that the lanes of
+// the segment accesses (PPW pairs, 64 / PPW consecutive k) fall on distinct banks as well.
+template <int N, int PPW>
+constexpr int pair_pitch = N + N / 16 + 64 / PPW;
+
+// The element `bytes` behind a wave-uniform base: a 32-bit lane offset on a scalar base, one
+// register where a 64-bit lane address takes two (the largest array here is 270 MB).
+template <typename V>
+__device__ __forceinline__ global_t<V>* at_bytes(global_t<V>* base, unsigned bytes) {
+    return reinterpret_cast<global_t<V>*>(reinterpret_cast<global_t<char>*>(base) + bytes);
+}
+template <typename V>
+__device__ __forceinline__ const global_t<V>* at_bytes(const global_t<V>* base, unsigned bytes) {
+    return reinterpret_cast<const global_t<V>*>(reinterpret_cast<const global_t<char>*>(base) + bytes);
+}
+
+// A pair of one wave needs no workgroup barrier in its own exchanges.
+template <int T>
+__device__ __forceinline__ void pair_sync( ) {
+    if constexpr ( T == 64 )
+        wave_lds_fence( );
+    else
+        __syncthreads( );
+}
+
+// u[r] times W_256^{j r} (conjugated for DIR > 0), j < 16, the second pass: table entries as
+// they are, 16 distinct addresses per load.
+template <int DIR>
+__device__ __forceinline__ void pair_twiddles_256(float2 (&u)[16], int j, const float2* __restrict__ twm) {
+    const auto* tab = as_global(twm) + 256;
+#pragma unroll
+    for ( int r = 1; r < 16; r++ ) {
+        const float2 w = load_cpx(at_bytes(tab, 8u * (unsigned)(j * r)), 0);
+        u[r]           = DIR < 0 ? cmul(u[r], w) : cmulc(u[r], w);
+    }
+}
+
+// Twiddles W_{Ns R}^{j r} of one thread's butterflies in the later passes, where a load's 64
+// addresses spread over 4 r cache lines: r = 4 a + b kept as the factors of 4 a and b (six
+// values for R = 16) and multiplied in one after the other.  (A table with every r's twiddles
+// contiguous in j measured 2-3 % slower, with the same errors against 64 bits.)
+template <int R, int B>
+struct PairTwiddles {
+    static constexpr int NB = R < 4 ? R : 4, NA = R / NB;
+    float2               lo[B][NB > 1 ? NB - 1 : 1], hi[B][NA > 1 ? NA - 1 : 1];
+
+    template <int Ns, int T>
+    __device__ __forceinline__ void load(int t, const float2* __restrict__ twm) {
+        const auto* tab = as_global(twm) + Ns * R;
+#pragma unroll
+        for ( int m = 0; m < B; m++ ) {
+            const int j = (t + T * m) & (Ns - 1);
+#pragma unroll
+            for ( int b = 1; b < NB; b++ )
+                lo[m][b - 1] = load_cpx(at_bytes(tab, 8u * (unsigned)(j * b)), 0);
+#pragma unroll
+            for ( int a = 1; a < NA; a++ )
+                hi[m][a - 1] = load_cpx(at_bytes(tab, 8u * (unsigned)(j * NB * a)), 0);
+        }
+    }
+
+    template <int DIR>
+    __device__ __forceinline__ void apply(float2 (&u)[R], int m) const {
+#pragma unroll
+        for ( int r = 1; r < R; r++ ) {
+            const int a = r / NB, b = r % NB;
+            if ( a )
+                u[r] = DIR < 0 ? cmul(u[r], hi[m][a - 1]) : cmulc(u[r], hi[m][a - 1]);
+            if ( b )
+                u[r] = DIR < 0 ? cmul(u[r], lo[m][b - 1]) : cmulc(u[r], lo[m][b - 1]);
+        }
+    }
+};
+
+// Stockham passes from stride Ns on: register i of thread t holds element t + T i on entry
+// and on return (natural order).  buf: the pair's N-float exchange buffer.
+template <int N, int Ns, int DIR>
+__device__ __forceinline__ void pair_passes(float2 (&v)[kPairE], float* __restrict__ buf, int t,
+                                            const float2* __restrict__ twm) {
+    constexpr int  T = N / kPairE, R = N / Ns < kPairE ? N / Ns : kPairE, B = kPairE / R;
+    constexpr bool LAST = Ns * R == N;
+    PairTwiddles<R, B> w;
+    if constexpr ( Ns > 16 )
+        w.template load<Ns, T>(t, twm);
+#pragma unroll
+    for ( int m = 0; m < B; m++ ) {
+        float2 u[R];
+#pragma unroll
+        for ( int r = 0; r < R; r++ )
+            u[r] = v[m + B * r];
+        if constexpr ( Ns == 16 )
+            pair_twiddles_256<DIR>(u, t & 15, twm);
+        else if constexpr ( Ns > 16 )
+            w.template apply<DIR>(u, m);
+        SmallDFT<R, DIR>::run(u);
+#pragma unroll
+        for ( int r = 0; r < R; r++ )
+            v[m + B * r] = u[r];
+    }
+    if constexpr ( ! LAST ) {
+        auto exchange = [&](auto part) {
+            pair_sync<T>( ); // the buffer's readers are done
+#pragma unroll
+            for ( int m = 0; m < B; m++ ) {
+                const int b = t + T * m, j = b & (Ns - 1);
+                float*    dst = buf + pair_slot((b - j) * R + j); // element (b - j) R + j + r Ns for r < R
+#pragma unroll
+                for ( int r = 0; r < R; r++ )
+                    dst[Ns == 1 ? r : r * pair_step(Ns)] = part(v[m + B * r]);
+            }
+            pair_sync<T>( );
+#pragma unroll
+            for ( int i = 0; i < kPairE; i++ )
+                part(v[i]) = buf[pair_slot(t) + i * pair_step(T)];
+        };
+        exchange([](float2& z) -> float& { return z.x; });
+        exchange([](float2& z) -> float& { return z.y; });
+        pair_passes<N, Ns * R, DIR>(v, buf, t, twm);
+    }
+}
+
+// R2C: rows 0 .. nlines - 1 of L real values (im.es = 1) into out[k om.es + row], k < nout
+// <= N/2 + 1; om.s1 = 1, om.es even, out 16-byte aligned, and om.es leaves room for an even
+// row count.  Grid: ceil(ceil(nlines / 2) / PPW) workgroups of T PPW threads.
+template <int N, int PPW, typename TIn>
+__global__ void __launch_bounds__(N / kPairE * PPW, N / kPairE * PPW == 1024 ? 8 : 4)
+        k_r2c_pair_rows(const TIn* __restrict__ in, LineMap im, int L, float2* __restrict__ out, LineMap om, int nout,
+                        int nlines, float pre_scale, const float2* __restrict__ tw) {
+    constexpr int T = N / kPairE, NT = T * PPW, H = N / 2, ITER = H / T + 1;
+    __shared__ float s_x[PPW * pair_pitch<N, PPW>];
+    const int     h     = PPW > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / T) : 0;
+    const int     t     = threadIdx.x % T;
+    const int     pair0 = xcd_row(blockIdx.x, gridDim.x) * PPW, row = 2 * (pair0 + h);
+    float*        buf   = s_x + h * pair_pitch<N, PPW>;
+    float2        v[kPairE];
+    {
+        const bool  ha = row < nlines, hb = row + 1 < nlines;
+        const auto* la = as_global(in) + im.base(ha ? row : 0);
+        const auto* lb = as_global(in) + im.base(hb ? row + 1 : 0);
+#pragma unroll
+        for ( int i = 0; i < kPairE; i++ ) {
+            const int n = t + T * i;
+            v[i]        = make_float2(0.f, 0.f);
+            if ( ha && n < L )
+                v[i].x = load_real(at_bytes(la, (unsigned)sizeof(TIn) * (unsigned)n), 0);
+            if ( hb && n < L )
+                v[i].y = load_real(at_bytes(lb, (unsigned)sizeof(TIn) * (unsigned)n), 0);
+        }
+#pragma unroll
+        for ( int i = 0; i < kPairE; i++ )
+            v[i] = cscale(v[i], pre_scale);
+    }
+    pair_passes<N, 1, -1>(v, buf, t, multi_twiddles(tw));
+    // Z in natural order through LDS, real parts first: item (k, g) takes A[k] and B[k] of the
+    // workgroup's pair g, 16 bytes of the segment of k
+    const int    g  = threadIdx.x % PPW, k0 = threadIdx.x / PPW; // k = k0 + T c
+    const float *zk = s_x + g * pair_pitch<N, PPW> + pair_slot(k0), *zn = s_x + g * pair_pitch<N, PPW> + pair_slot(N - k0);
+    float        ax[ITER], by[ITER];
+    auto         spread = [&](auto part) {
+        __syncthreads( );
+#pragma unroll
+        for ( int i = 0; i < kPairE; i++ )
+            buf[pair_slot(t) + i * pair_step(T)] = part(v[i]);
+        if ( t == 0 )
+            buf[pair_step(N)] = part(v[0]);
+        __syncthreads( );
+    };
+    spread([](float2 z) { return z.x; });
+#pragma unroll
+    for ( int c = 0; c < ITER; c++ )
+        if ( c + 1 < ITER || k0 == 0 ) {
+            ax[c] = 0.5f * (zk[c * pair_step(T)] + zn[-c * pair_step(T)]);
+            by[c] = 0.5f * (zn[-c * pair_step(T)] - zk[c * pair_step(T)]);
+        }
+    spread([](float2 z) { return z.y; });
+    auto*      op   = as_global(out) + 2 * pair0;
+    const bool rows = 2 * (pair0 + g) < nlines;
+#pragma unroll
+    for ( int c = 0; c < ITER; c++ ) {
+        const int k = k0 + T * c;
+        if ( k < nout && rows && (c + 1 < ITER || k0 == 0) ) {
+            const float yk = zk[c * pair_step(T)], yn = zn[-c * pair_step(T)];
+            store_cpx_pair(at_bytes(op, 8u * (unsigned)k * (unsigned)om.es + 16u * (unsigned)g), 0,
+                           make_float2(ax[c], 0.5f * (yk - yn)), make_float2(0.5f * (yk + yn), by[c]));
+        }
+    }
+}
+
+// C2R: in[k im.es + row], k <= N/2 (im.s1 = 1, im.es even, in 16-byte aligned), to the
+// window y[(o + j) mod N], j < M, of every row (om.es = 1).  The imaginary parts of
+// k = 0 and N/2 are dropped, as the real part of the Hermitian extension's inverse drops
+// them.  Grid as above.
+template <int N, int PPW, typename TOut>
+__global__ void __launch_bounds__(N / kPairE * PPW, N / kPairE * PPW == 1024 ? 8 : 4)
+        k_c2r_pair_rows(const float2* __restrict__ in, LineMap im, TOut* __restrict__ out, LineMap om, int M, int o,
+                        int nlines, float post_scale, const float2* __restrict__ tw) {
+    constexpr int T = N / kPairE, NT = T * PPW, H = N / 2, ITER = H / T + 1;
+    __shared__ float s_x[PPW * pair_pitch<N, PPW>];
+    const int     h     = PPW > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / T) : 0;
+    const int     t     = threadIdx.x % T;
+    const int     pair0 = xcd_row(blockIdx.x, gridDim.x) * PPW, row = 2 * (pair0 + h);
+    float*        buf   = s_x + h * pair_pitch<N, PPW>;
+    float2        v[kPairE];
+    {
+        const auto* ip   = as_global(in) + 2 * pair0;
+        const int   g    = threadIdx.x % PPW, k0 = threadIdx.x / PPW; // k = k0 + T c
+        const bool  ha   = 2 * (pair0 + g) < nlines, hb = 2 * (pair0 + g) + 1 < nlines;
+        float4      u[ITER];
+#pragma unroll
+        for ( int c = 0; c < ITER; c++ ) {
+            const int k = k0 + T * c;
+            u[c]        = make_float4(0.f, 0.f, 0.f, 0.f);
+            if ( ha && (c + 1 < ITER || k0 == 0) )
+                u[c] = load_cpx_pair(at_bytes(ip, 8u * (unsigned)k * (unsigned)im.es + 16u * (unsigned)g), 0);
+            if ( ! hb ) // past the last row: whatever the buffer holds
+                u[c].z = u[c].w = 0.f;
+            if ( (c == 0 || c + 1 == ITER) && k0 == 0 )
+                u[c].y = u[c].w = 0.f;
+        }
+        float *zk = s_x + g * pair_pitch<N, PPW> + pair_slot(k0), *zn = s_x + g * pair_pitch<N, PPW> + pair_slot(N - k0);
+        auto   spread = [&](auto lo, auto hi) {
+#pragma unroll
+            for ( int c = 0; c < ITER; c++ )
+                if ( c + 1 < ITER || k0 == 0 ) { // (element N / 2 is its own mirror, and lo = hi there)
+                    zk[c * pair_step(T)]  = lo(u[c]);
+                    zn[-c * pair_step(T)] = hi(u[c]);
+                }
+            __syncthreads( );
+        };
+        spread([](float4 z) { return z.x - z.w; }, [](float4 z) { return z.x + z.w; });
+#pragma unroll
+        for ( int i = 0; i < kPairE; i++ )
+            v[i].x = buf[pair_slot(t) + i * pair_step(T)];
+        __syncthreads( );
+        spread([](float4 z) { return z.z + z.y; }, [](float4 z) { return z.z - z.y; });
+#pragma unroll
+        for ( int i = 0; i < kPairE; i++ )
+            v[i].y = buf[pair_slot(t) + i * pair_step(T)];
+    }
+    __syncthreads( ); // (the first exchange of a one-wave pair orders its own wave only)
+    pair_passes<N, 1, +1>(v, buf, t, multi_twiddles(tw));
+    if ( row >= nlines )
+        return;
+    const bool hb = row + 1 < nlines;
+    auto*      oa = as_global(out) + om.base(row);
+    auto*      ob = as_global(out) + om.base(hb ? row + 1 : row);
+#pragma unroll
+    for ( int i = 0; i < kPairE; i++ ) {
+        const int j = (t + T * i - o) & (N - 1);
+        if ( j < M ) {
+            store_real(at_bytes(oa, (unsigned)sizeof(TOut) * (unsigned)j), 0, v[i].x * post_scale);
+            if ( hb )
+                store_real(at_bytes(ob, (unsigned)sizeof(TOut) * (unsigned)j), 0, v[i].y * post_scale);
+        }
+    }
+}
+
+} // namespace fastfft_amd

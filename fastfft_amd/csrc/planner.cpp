@@ -162,6 +162,13 @@ static long ws_ld(int n) {
     return n + pad;
 }
 
+// Leading dimension of a workspace array of columns (2-D FwdFFT and InvFFT: A[kx][y]) of n
+// values: a multiple of 8, so that the 64-byte segments that the x-passes move (eight
+// neighbouring rows of one kx) are aligned, and an odd row count has its partner's slot.
+static long ws_ld_columns(int n) {
+    return (ws_ld(n) + 7) / 8 * 8;
+}
+
 // Leading dimension of a row-major workspace array of n complex values per row:
 // even, so that every row starts 16-byte aligned for the 16-byte row accesses.
 static long ws_ld_rows(int n) {
@@ -211,7 +218,7 @@ static PlanError fwd_stages_2d(const PlanState& p, std::vector<Stage>& st, Buf f
     s1.im       = lm(pitch, 0, 1, 1);
     s1.dst      = Buf::ws_a;
     s1.dst_elem = Elem::cpx_f32;
-    s1.om       = lm(1, 0, ws_ld(in.y), 1);
+    s1.om       = lm(1, 0, ws_ld_columns(in.y), 1);
     st.push_back(s1);
     // y-pass: each of the out.w columns A[kx][0..in.y) -> C[kx][ky]
     const int Ny = std::max(in.y, out.y);
@@ -220,7 +227,7 @@ static PlanError fwd_stages_2d(const PlanState& p, std::vector<Stage>& st, Buf f
                               Ny, in.y, 0, 0, out.y, out.w);
     s2.src      = Buf::ws_a;
     s2.src_elem = Elem::cpx_f32;
-    s2.im       = lm(ws_ld(in.y), 0, 1, 1);
+    s2.im       = lm(ws_ld_columns(in.y), 0, 1, 1);
     s2.dst      = final_dst;
     s2.dst_elem = Elem::cpx_input_type;
     s2.om       = lm(out.y, 0, 1, 1);
@@ -288,14 +295,14 @@ static PlanError inv_stages_2d(const PlanState& p, std::vector<Stage>& st, Buf s
     s1.im       = lm(in.y, 0, 1, 1);
     s1.dst      = Buf::ws_b;
     s1.dst_elem = Elem::cpx_f32;
-    s1.om       = lm(ws_ld(out.y), 0, 1, 1);
+    s1.om       = lm(ws_ld_columns(out.y), 0, 1, 1);
     st.push_back(s1);
     // x-pass C2R on the out.y rows -> out[j][pitch]
     Stage s2    = make_stage(StageKind::inv_c2r, dec ? "c2r_decrease_XY" : "c2r_none_XY", in.x, 0, out.x,
                              axis_origin(p, 0, in.x, out.x), 0, out.y);
     s2.src      = Buf::ws_b;
     s2.src_elem = Elem::cpx_f32;
-    s2.im       = lm(1, 0, ws_ld(out.y), 1);
+    s2.im       = lm(1, 0, ws_ld_columns(out.y), 1);
     s2.dst      = Buf::user_out;
     s2.dst_elem = Elem::real_input_type;
     s2.om       = lm(2 * out.w, 0, 1, 1);
@@ -520,6 +527,12 @@ void stage_list_workspace(const std::vector<Stage>& st, size_t& ws_a, size_t& ws
     for ( const Stage& s : st ) {
         int    nw = s.kind == StageKind::fwd_real || s.kind == StageKind::fwd_cpx ? s.nout : s.M;
         size_t ex = extent(s.om, s.nlines, nw);
+        // arrays of columns (2-D x- and y-passes) are read and written in segments of rows: whole
+        // columns, the padding of the last one included
+        if ( s.om.n2 == 1 && s.kind == StageKind::fwd_real && s.om.s1 == 1 && s.om.es > 1 )
+            ex = std::max(ex, (size_t)nw * (size_t)s.om.es);
+        if ( s.om.n2 == 1 && s.kind == StageKind::inv_cpx && s.om.es == 1 )
+            ex = std::max(ex, (size_t)s.nlines * (size_t)s.om.s1);
         if ( s.dst == Buf::ws_a )
             ws_a = std::max(ws_a, ex);
         if ( s.dst == Buf::ws_b )
