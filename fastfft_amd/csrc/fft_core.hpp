@@ -131,6 +131,17 @@ __device__ __forceinline__ global_t<T>* as_global(T* p) {
     return (global_t<T>*)p;
 }
 
+// The element `bytes` behind a wave-uniform base: a 32-bit lane offset on a scalar base, one
+// register where a 64-bit lane address takes two (for arrays below 4 GiB).
+template <typename V>
+__device__ __forceinline__ global_t<V>* at_bytes(global_t<V>* base, unsigned bytes) {
+    return reinterpret_cast<global_t<V>*>(reinterpret_cast<global_t<char>*>(base) + bytes);
+}
+template <typename V>
+__device__ __forceinline__ const global_t<V>* at_bytes(const global_t<V>* base, unsigned bytes) {
+    return reinterpret_cast<const global_t<V>*>(reinterpret_cast<const global_t<char>*>(base) + bytes);
+}
+
 // Launch descriptors, read-only while a kernel runs and read at wave-uniform
 // addresses, are read through the constant address space: scalar loads into
 // scalar registers.
@@ -198,6 +209,22 @@ __device__ __forceinline__ void store_cpx(global_t<__half2>* p, long i, float2 v
     const unsigned lo = __half_as_ushort(__float2half_rn(v.x)), hi = __half_as_ushort(__float2half_rn(v.y));
     reinterpret_cast<global_t<unsigned>*>(p)[i] = lo | (hi << 16);
 }
+
+// An element's bits as loaded and their FP32 value apart: predicated loads of a thread stay in
+// flight together only if nothing in their branches uses the values.
+__device__ __forceinline__ float          load_bits(const global_t<float>* p) { return *p; }
+__device__ __forceinline__ unsigned short load_bits(const global_t<__half>* p) { return *reinterpret_cast<const global_t<unsigned short>*>(p); }
+__device__ __forceinline__ gvec2          load_bits(const global_t<float2>* p) { return *reinterpret_cast<const global_t<gvec2>*>(p); }
+__device__ __forceinline__ unsigned       load_bits(const global_t<__half2>* p) { return *reinterpret_cast<const global_t<unsigned>*>(p); }
+__device__ __forceinline__ float          bits_value(float v) { return v; }
+__device__ __forceinline__ float          bits_value(unsigned short v) { return __half2float(__ushort_as_half(v)); }
+__device__ __forceinline__ float2         bits_value(gvec2 v) { return make_float2(v.x, v.y); }
+__device__ __forceinline__ float2         bits_value(unsigned v) {
+    return make_float2(__half2float(__ushort_as_half((unsigned short)(v & 0xffffu))),
+                       __half2float(__ushort_as_half((unsigned short)(v >> 16))));
+}
+template <typename T>
+using bits_t = decltype(load_bits((const global_t<T>*)nullptr));
 
 // elements 2 m and 2 m + 1 of an 8-byte aligned line of half pairs
 __device__ __forceinline__ void store_cpx_pair(global_t<__half2>* p, long m, float2 a, float2 b) {

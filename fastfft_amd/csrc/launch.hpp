@@ -58,11 +58,11 @@ struct StageIO {
 bool       r2c_rows_batch_covers(const Stage& s);
 bool       c2r_rows_batch_covers(const Stage& s);
 bool       xcorr_col_covers(const Stage& s, CpxT img_ct);
-// complex forward / inverse line stages over adjacent lines with far-apart
-// elements (3-D z-passes), N = 256 or 512: tiled kernel (tile_lines.hpp);
+// line stages of 64 to 512 points whose lines are unit stride or lie next to each other
+// (lines.hpp): 3-D passes, the 256- and 512-point passes of 2-D transforms, the fused z-pass;
 // hipErrorNotSupported, before launching anything, when it does not cover s
-bool       tile_lines_cover(const Stage& s);
-hipError_t launch_tile_lines(const Stage& s, const StageIO& io, const float2* tw, hipStream_t stream);
+bool       lines_cover(const Stage& s);
+hipError_t launch_lines(const Stage& s, const StageIO& io, const float2* tw, hipStream_t stream);
 // the split-BF16 matrix-core correlation pass (xcorr_toeplitz.hpp) on a frame in mixed
 // form: N = 1024, L <= 512, M <= 512, L + M - 1 <= 1024, window origin 0, the DC and
 // Nyquist columns of a real transform at both ends, row-major template and output

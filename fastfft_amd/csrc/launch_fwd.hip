@@ -258,6 +258,13 @@ hipError_t launch_fwd(const Stage& s, const StageIO& io, const float2* tw, hipSt
         if ( e != hipErrorNotSupported )
             return e;
     }
+    // lines of 64 to 512 points: C2C passes, and real rows into a transposed spectrum
+    if ( (s.kind == StageKind::fwd_cpx || (s.kind == StageKind::fwd_real && s.om.es != 1)) &&
+         ! env_int("FASTFFT_NO_WAVE_ROWS", 0) ) {
+        hipError_t e = launch_lines(s, io, tw, st);
+        if ( e != hipErrorNotSupported )
+            return e;
+    }
     if ( io.src_real && ! io.dst_real && io.dst_ct == CpxT::c64 && ! env_int("FASTFFT_NO_WAVE_ROWS", 0) ) {
         hipError_t e = launch_r2c_packed(s, io.src, io.dst, io.src_rt, s.nlines, io.scale, tw, nullptr, 1, st);
         if ( e != hipErrorNotSupported )
@@ -268,15 +275,7 @@ hipError_t launch_fwd(const Stage& s, const StageIO& io, const float2* tw, hipSt
         if ( e != hipErrorNotSupported )
             return e;
     }
-    // C2C passes, and real rows whose spectra are stored transposed (a 3-D x-pass): 16 lines per
-    // workgroup, transposed through LDS into 128-byte segments
-    if ( (s.kind == StageKind::fwd_cpx || (s.kind == StageKind::fwd_real && s.om.es != 1)) &&
-         ! env_int("FASTFFT_NO_WAVE_ROWS", 0) ) {
-        hipError_t e = launch_tile_lines(s, io, tw, st);
-        if ( e != hipErrorNotSupported )
-            return e;
-    }
-    // padded lines the tiles leave: unit-stride complex lines, and real rows into a transposed
+    // padded lines left: unit-stride complex lines, and real rows into a transposed
     // spectrum that no sub-transform kernel takes
     if ( full_lines && s.L < s.N && (io.src_real ? s.om.es != 1 && ! r2c_rows_shape(s) : s.im.es == 1 && s.om.es == 1) ) {
         hipError_t e = try_full_wave(s, io, tw, st);

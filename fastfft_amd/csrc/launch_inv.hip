@@ -151,14 +151,6 @@ hipError_t launch_stats_reset(const BatchStats& bs, long n, hipStream_t st) {
 static hipError_t try_c2r_packed(const Stage& s, const StageIO& io, const float2* tw, hipStream_t st) {
     if ( ! c2r_packed_covers(s) || io.src_real || io.src_ct != CpxT::c64 || ! io.dst_real )
         return hipErrorNotSupported;
-    // rows whose elements lie far apart (a 3-D inverse's x-pass, a 2-D InvFFT's 512-point rows):
-    // the tiled line kernel reads 16 neighbouring rows per 128-byte access, where one wave per
-    // row would gather 8 bytes per element
-    if ( s.im.es != 1 && ! io.amax && ! env_int("FASTFFT_NO_TILE_LINES", 0) ) {
-        const hipError_t e = launch_tile_lines(s, io, tw, st);
-        if ( e != hipErrorNotSupported )
-            return e;
-    }
     const bool keys = io.amax && s.nlines <= kArgmaxPartials;
     hipError_t e    = launch_c2r_packed(s, io.src, io.dst, io.dst_rt, io.scale, tw, keys ? io.amax->keys : nullptr,
                                         nullptr, 1, st);
@@ -514,6 +506,9 @@ static hipError_t try_c2r_pair_rows(const Stage& s, const StageIO& io, const flo
 hipError_t launch_inv(const Stage& s, const StageIO& io, const float2* tw, hipStream_t st) {
     if ( ! env_int("FASTFFT_NO_WAVE_ROWS", 0) ) {
         hipError_t e = try_c2r_pair_rows(s, io, tw, st);
+        // lines of 64 to 512 points (a C2R pass asked for its argmax keeps the row kernels)
+        if ( e == hipErrorNotSupported && ! io.amax )
+            e = launch_lines(s, io, tw, st);
         if ( e == hipErrorNotSupported )
             e = try_c2r_packed(s, io, tw, st);
         if ( e == hipErrorNotSupported )
@@ -523,12 +518,6 @@ hipError_t launch_inv(const Stage& s, const StageIO& io, const float2* tw, hipSt
     }
     if ( ! env_int("FASTFFT_NO_WAVE_ROWS", 0) && ! env_int("FASTFFT_NO_FULL_LINES", 0) && ! io.amax ) {
         hipError_t e = try_full_inv(s, io, tw, st);
-        if ( e != hipErrorNotSupported )
-            return e;
-    }
-    // 256 / 512-point lines, 16 per workgroup (a C2R pass asked for its argmax keeps the row kernel)
-    if ( (s.kind == StageKind::inv_cpx || (s.kind == StageKind::inv_c2r && ! io.amax)) && ! env_int("FASTFFT_NO_WAVE_ROWS", 0) ) {
-        hipError_t e = launch_tile_lines(s, io, tw, st);
         if ( e != hipErrorNotSupported )
             return e;
     }

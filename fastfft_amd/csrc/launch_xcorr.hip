@@ -158,9 +158,14 @@ hipError_t launch_xcorr(const Stage& s, const StageIO& io, const float2* tw, hip
         if ( e != hipErrorNotSupported )
             return e;
     }
-    // the generic kernel correlates one template per launch
+    // the kernels below correlate one template per launch
     if ( io.xitems )
         return hipErrorNotSupported;
+    if ( ! env_int("FASTFFT_NO_WAVE_ROWS", 0) ) {
+        hipError_t e = launch_lines(s, io, tw, st);
+        if ( e != hipErrorNotSupported )
+            return e;
+    }
     return dispatch_P(s.P, [&](auto pc) -> hipError_t {
         constexpr int P = decltype(pc)::value;
         if ( io.img_ct == CpxT::c64 )

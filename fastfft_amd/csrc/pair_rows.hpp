@@ -36,17 +36,6 @@ constexpr int                  pair_step(int k) { return k + k / 16; }
 template <int N, int PPW>
 constexpr int pair_pitch = N + N / 16 + 64 / PPW;
 
-// The element `bytes` behind a wave-uniform base: a 32-bit lane offset on a scalar base, one
-// register where a 64-bit lane address takes two (the largest array here is 270 MB).
-template <typename V>
-__device__ __forceinline__ global_t<V>* at_bytes(global_t<V>* base, unsigned bytes) {
-    return reinterpret_cast<global_t<V>*>(reinterpret_cast<global_t<char>*>(base) + bytes);
-}
-template <typename V>
-__device__ __forceinline__ const global_t<V>* at_bytes(const global_t<V>* base, unsigned bytes) {
-    return reinterpret_cast<const global_t<V>*>(reinterpret_cast<const global_t<char>*>(base) + bytes);
-}
-
 // A pair of one wave needs no workgroup barrier in its own exchanges.
 template <int T>
 __device__ __forceinline__ void pair_sync( ) {
@@ -170,18 +159,20 @@ __global__ void __launch_bounds__(N / kPairE * PPW, N / kPairE * PPW == 1024 ? 8
         const bool  ha = row < nlines, hb = row + 1 < nlines;
         const auto* la = as_global(in) + im.base(ha ? row : 0);
         const auto* lb = as_global(in) + im.base(hb ? row + 1 : 0);
+        // every load of the thread in flight before the first value is used
+        bits_t<TIn> a[kPairE], b[kPairE];
 #pragma unroll
         for ( int i = 0; i < kPairE; i++ ) {
             const int n = t + T * i;
-            v[i]        = make_float2(0.f, 0.f);
+            a[i] = b[i] = bits_t<TIn>{ };
             if ( ha && n < L )
-                v[i].x = load_real(at_bytes(la, (unsigned)sizeof(TIn) * (unsigned)n), 0);
+                a[i] = load_bits(at_bytes(la, (unsigned)sizeof(TIn) * (unsigned)n));
             if ( hb && n < L )
-                v[i].y = load_real(at_bytes(lb, (unsigned)sizeof(TIn) * (unsigned)n), 0);
+                b[i] = load_bits(at_bytes(lb, (unsigned)sizeof(TIn) * (unsigned)n));
         }
 #pragma unroll
         for ( int i = 0; i < kPairE; i++ )
-            v[i] = cscale(v[i], pre_scale);
+            v[i] = make_float2(bits_value(a[i]) * pre_scale, bits_value(b[i]) * pre_scale);
     }
     pair_passes<N, 1, -1>(v, buf, t, multi_twiddles(tw));
     // Z in natural order through LDS, real parts first: item (k, g) takes A[k] and B[k] of the
@@ -245,6 +236,9 @@ __global__ void __launch_bounds__(N / kPairE * PPW, N / kPairE * PPW == 1024 ? 8
             u[c]        = make_float4(0.f, 0.f, 0.f, 0.f);
             if ( ha && (c + 1 < ITER || k0 == 0) )
                 u[c] = load_cpx_pair(at_bytes(ip, 8u * (unsigned)k * (unsigned)im.es + 16u * (unsigned)g), 0);
+        }
+#pragma unroll
+        for ( int c = 0; c < ITER; c++ ) {
             if ( ! hb ) // past the last row: whatever the buffer holds
                 u[c].z = u[c].w = 0.f;
             if ( (c == 0 || c + 1 == ITER) && k0 == 0 )
