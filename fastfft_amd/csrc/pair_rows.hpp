@@ -14,8 +14,8 @@
 // imaginary parts through one LDS buffer of N floats per pair.  That halves the LDS of a
 // pair, and immediate offsets keep the addresses out of the registers (64 at most), so two
 // workgroups of 1024 threads share a CU and one loads or stores while the other computes.
-// Bound by arithmetic and memory about alike: 4096^2 (134 MB) takes 30.7 us forward and
-// 29.7 us inverse, 4.4-4.5 TB/s, where complex exchanges with one workgroup per CU took
+// Bound by arithmetic and memory about alike: 4096^2 (134 MB) takes 29.9 us forward and
+// 29.7 us inverse, 4.5 TB/s, where complex exchanges with one workgroup per CU took
 // 38.6 us forward and one row per workgroup with 8-byte gathers 51.7 us inverse.
 #pragma once
 
@@ -45,17 +45,31 @@ __device__ __forceinline__ void pair_sync( ) {
         __syncthreads( );
 }
 
-// u[r] times W_256^{j r} (conjugated for DIR > 0), j < 16, the second pass: table entries as
-// they are, 16 distinct addresses per load.
-template <int DIR>
-__device__ __forceinline__ void pair_twiddles_256(float2 (&u)[16], int j, const float2* __restrict__ twm) {
-    const auto* tab = as_global(twm) + 256;
+// The second pass's twiddles W_256^{j r}, [r - 1][j], copied into LDS once per workgroup of NT
+// threads (read from memory at their use instead, 4096^2 takes 59.0 us forward and 33.9 us cut
+// to 1001 x 900, here 57.2 and 32.4): load() issues the thread's loads, store() writes them.
+constexpr int kPairTable = 15 * 16;
+template <int NT>
+struct PairTable {
+    static constexpr int ROWS = (kPairTable + NT - 1) / NT;
+    float2               w[ROWS];
+    __device__ __forceinline__ void load(const float2* __restrict__ twm) {
 #pragma unroll
-    for ( int r = 1; r < 16; r++ ) {
-        const float2 w = load_cpx(at_bytes(tab, 8u * (unsigned)(j * r)), 0);
-        u[r]           = DIR < 0 ? cmul(u[r], w) : cmulc(u[r], w);
+        for ( int r = 0; r < ROWS; r++ ) {
+            const int g = threadIdx.x + NT * r;
+            if ( g < kPairTable )
+                w[r] = load_cpx(as_global(twm), 256 + (g & 15) * (1 + (g >> 4)));
+        }
     }
-}
+    __device__ __forceinline__ void store(float2* tab) const {
+#pragma unroll
+        for ( int r = 0; r < ROWS; r++ ) {
+            const int g = threadIdx.x + NT * r;
+            if ( g < kPairTable )
+                tab[g] = w[r];
+        }
+    }
+};
 
 // Twiddles W_{Ns R}^{j r} of one thread's butterflies in the later passes, where a load's 64
 // addresses spread over 4 r cache lines: r = 4 a + b kept as the factors of 4 a and b (six
@@ -98,7 +112,7 @@ struct PairTwiddles {
 // and on return (natural order).  buf: the pair's N-float exchange buffer.
 template <int N, int Ns, int DIR>
 __device__ __forceinline__ void pair_passes(float2 (&v)[kPairE], float* __restrict__ buf, int t,
-                                            const float2* __restrict__ twm) {
+                                            const float2* tab, const float2* __restrict__ twm) {
     constexpr int  T = N / kPairE, R = N / Ns < kPairE ? N / Ns : kPairE, B = kPairE / R;
     constexpr bool LAST = Ns * R == N;
     PairTwiddles<R, B> w;
@@ -110,8 +124,13 @@ __device__ __forceinline__ void pair_passes(float2 (&v)[kPairE], float* __restri
 #pragma unroll
         for ( int r = 0; r < R; r++ )
             u[r] = v[m + B * r];
-        if constexpr ( Ns == 16 )
-            pair_twiddles_256<DIR>(u, t & 15, twm);
+        if constexpr ( Ns == 16 ) {
+#pragma unroll
+            for ( int r = 1; r < R; r++ ) {
+                const float2 w2 = tab[(r - 1) * 16 + (t & 15)];
+                u[r]            = DIR < 0 ? cmul(u[r], w2) : cmulc(u[r], w2);
+            }
+        }
         else if constexpr ( Ns > 16 )
             w.template apply<DIR>(u, m);
         SmallDFT<R, DIR>::run(u);
@@ -137,7 +156,7 @@ __device__ __forceinline__ void pair_passes(float2 (&v)[kPairE], float* __restri
         };
         exchange([](float2& z) -> float& { return z.x; });
         exchange([](float2& z) -> float& { return z.y; });
-        pair_passes<N, Ns * R, DIR>(v, buf, t, twm);
+        pair_passes<N, Ns * R, DIR>(v, buf, t, tab, twm);
     }
 }
 
@@ -149,7 +168,10 @@ __global__ void __launch_bounds__(N / kPairE * PPW, N / kPairE * PPW == 1024 ? 8
         k_r2c_pair_rows(const TIn* __restrict__ in, LineMap im, int L, float2* __restrict__ out, LineMap om, int nout,
                         int nlines, float pre_scale, const float2* __restrict__ tw) {
     constexpr int T = N / kPairE, NT = T * PPW, H = N / 2, ITER = H / T + 1;
-    __shared__ float s_x[PPW * pair_pitch<N, PPW>];
+    __shared__ float  s_x[PPW * pair_pitch<N, PPW>];
+    __shared__ float2 s_tw[kPairTable];
+    PairTable<NT>     table;
+    table.load(multi_twiddles(tw));
     const int     h     = PPW > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / T) : 0;
     const int     t     = threadIdx.x % T;
     const int     pair0 = xcd_row(blockIdx.x, gridDim.x) * PPW, row = 2 * (pair0 + h);
@@ -174,7 +196,9 @@ __global__ void __launch_bounds__(N / kPairE * PPW, N / kPairE * PPW == 1024 ? 8
         for ( int i = 0; i < kPairE; i++ )
             v[i] = make_float2(bits_value(a[i]) * pre_scale, bits_value(b[i]) * pre_scale);
     }
-    pair_passes<N, 1, -1>(v, buf, t, multi_twiddles(tw));
+    table.store(s_tw);
+    __syncthreads( );
+    pair_passes<N, 1, -1>(v, buf, t, s_tw, multi_twiddles(tw));
     // Z in natural order through LDS, real parts first: item (k, g) takes A[k] and B[k] of the
     // workgroup's pair g, 16 bytes of the segment of k
     const int    g  = threadIdx.x % PPW, k0 = threadIdx.x / PPW; // k = k0 + T c
@@ -219,7 +243,10 @@ __global__ void __launch_bounds__(N / kPairE * PPW, N / kPairE * PPW == 1024 ? 8
         k_c2r_pair_rows(const float2* __restrict__ in, LineMap im, TOut* __restrict__ out, LineMap om, int M, int o,
                         int nlines, float post_scale, const float2* __restrict__ tw) {
     constexpr int T = N / kPairE, NT = T * PPW, H = N / 2, ITER = H / T + 1;
-    __shared__ float s_x[PPW * pair_pitch<N, PPW>];
+    __shared__ float  s_x[PPW * pair_pitch<N, PPW>];
+    __shared__ float2 s_tw[kPairTable];
+    PairTable<NT>     table;
+    table.load(multi_twiddles(tw));
     const int     h     = PPW > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / T) : 0;
     const int     t     = threadIdx.x % T;
     const int     pair0 = xcd_row(blockIdx.x, gridDim.x) * PPW, row = 2 * (pair0 + h);
@@ -245,6 +272,7 @@ __global__ void __launch_bounds__(N / kPairE * PPW, N / kPairE * PPW == 1024 ? 8
                 u[c].y = u[c].w = 0.f;
         }
         float *zk = s_x + g * pair_pitch<N, PPW> + pair_slot(k0), *zn = s_x + g * pair_pitch<N, PPW> + pair_slot(N - k0);
+        table.store(s_tw);
         auto   spread = [&](auto lo, auto hi) {
 #pragma unroll
             for ( int c = 0; c < ITER; c++ )
@@ -265,7 +293,7 @@ __global__ void __launch_bounds__(N / kPairE * PPW, N / kPairE * PPW == 1024 ? 8
             v[i].y = buf[pair_slot(t) + i * pair_step(T)];
     }
     __syncthreads( ); // (the first exchange of a one-wave pair orders its own wave only)
-    pair_passes<N, 1, +1>(v, buf, t, multi_twiddles(tw));
+    pair_passes<N, 1, +1>(v, buf, t, s_tw, multi_twiddles(tw));
     if ( row >= nlines )
         return;
     const bool hb = row + 1 < nlines;
