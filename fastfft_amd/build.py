@@ -27,7 +27,7 @@ SOURCES = ["planner.cpp", "capi.cpp", "launch_fwd.hip", "launch_inv.hip", "launc
            "tuning.cpp"]
 HEADERS = ["fft_core.hpp", "line_kernels.hpp", "launch.hpp", "launch_common.hpp", "plan.hpp", "wave_fft.hpp",
            "xcorr_col.hpp", "rows_wave.hpp", "items.hpp", "full_wave.hpp", "window_rows.hpp", "xcorr_toeplitz.hpp", "rows_packed.hpp",
-           "pair_rows.hpp", "lines.hpp", "tuning.hpp"]
+           "pair_rows.hpp", "lines.hpp", "xcorr_one.hpp", "tuning.hpp"]
 
 
 def _needs(obj: str, src: str) -> bool:

@@ -67,6 +67,18 @@ static hipError_t launch_r2c_packed(const Stage& s, const void* src, void* dst, 
                             : go_r2c_packed<512, __half>(s, src, dst, nrows, pre, tw, items, n, st);
 }
 
+// The stage with sub-transforms of at least 256 points: shorter ones run no faster per point,
+// and no row kernel takes them (128 of 2048 points: the whole correlation 40 us on the generic
+// line kernel).
+static Stage r2c_at_least_256(const Stage& s) {
+    Stage r = s;
+    if ( r.P < 256 && r.N >= 256 ) {
+        r.P = 256;
+        r.Q = r.N / 256;
+    }
+    return r;
+}
+
 // (P, Q) of an R2C row stage that k_r2c_rows_wave covers
 static bool r2c_rows_shape(const Stage& s) {
     return (s.P == 256 || s.P == 512 || s.P == 1024) && (s.Q == 1 || s.Q == 2 || s.Q == 4 || s.Q == 8 || s.Q == 16) &&
@@ -275,15 +287,15 @@ hipError_t launch_fwd(const Stage& s, const StageIO& io, const float2* tw, hipSt
         if ( e != hipErrorNotSupported )
             return e;
     }
-    // padded lines left: unit-stride complex lines, and real rows into a transposed
-    // spectrum that no sub-transform kernel takes
-    if ( full_lines && s.L < s.N && (io.src_real ? s.om.es != 1 && ! r2c_rows_shape(s) : s.im.es == 1 && s.om.es == 1) ) {
+    // padded lines left: unit-stride complex lines, and real rows that no sub-transform kernel takes
+    if ( full_lines && s.L < s.N && (io.src_real ? ! r2c_rows_shape(r2c_at_least_256(s)) : s.im.es == 1 && s.om.es == 1) ) {
         hipError_t e = try_full_wave(s, io, tw, st);
         if ( e != hipErrorNotSupported )
             return e;
     }
     if ( io.src_real && ! io.dst_real && io.dst_ct == CpxT::c64 && rows_ok && ! env_int("FASTFFT_NO_WAVE_ROWS", 0) ) {
-        hipError_t e = io.src_rt == RealT::f32 ? try_r2c_wave<float>(s, io, tw, st) : try_r2c_wave<__half>(s, io, tw, st);
+        const Stage r = r2c_at_least_256(s);
+        hipError_t  e = io.src_rt == RealT::f32 ? try_r2c_wave<float>(r, io, tw, st) : try_r2c_wave<__half>(r, io, tw, st);
         if ( e != hipErrorNotSupported )
             return e;
     }

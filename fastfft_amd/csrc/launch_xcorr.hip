@@ -10,6 +10,7 @@
 
 #include "launch_common.hpp"
 #include "xcorr_col.hpp"
+#include "xcorr_one.hpp"
 #include "xcorr_toeplitz.hpp"
 
 namespace fastfft_amd {
@@ -50,12 +51,7 @@ static hipError_t go_xcorr_col(const Stage& s, const StageIO& io, const float2* 
     }
     XcorrItem one{io.src, io.dst, s.L, 0};
     const dim3 grid((unsigned)blocks, (unsigned)groups), block(64 * Q);
-    // one template per launch: the single-template form (FASTFFT_XCORR_ONE=0 keeps the loop form)
-    if ( ! io.xitems && env_int("FASTFFT_XCORR_ONE", 1) )
-        launch_kernel<k_xcorr_col<P, Q, RS, TImg, true>>(grid, block, 0, st, one, nullptr, 1, s.im.s1, s.im.es,
-                static_cast<const TImg*>(io.img), s.gm.s1, s.om.s1, s.om.es, s.M, s.o, io.scale, tw, s.nlines - 1, pack);
-    else
-        launch_kernel<k_xcorr_col<P, Q, RS, TImg>>(grid, block, 0, st, one, static_cast<const XcorrItem*>(io.xitems),
+    launch_kernel<k_xcorr_col<P, Q, RS, TImg>>(grid, block, 0, st, one, static_cast<const XcorrItem*>(io.xitems),
                 io.nxitems, s.im.s1, s.im.es, static_cast<const TImg*>(io.img), s.gm.s1, s.om.s1, s.om.es, s.M, s.o, io.scale,
                 tw, s.nlines - 1, pack);
     return hipGetLastError( );
@@ -86,6 +82,30 @@ static hipError_t try_xcorr_col(const Stage& s, const StageIO& io, const float2*
         case 4: return by_q(std::integral_constant<int, 4>{ });
         case 8: return by_q(std::integral_constant<int, 8>{ });
         case 16: return by_q(std::integral_constant<int, 16>{ });
+        default: return hipErrorNotSupported;
+    }
+}
+
+// One template, any length, window and origin: one workgroup per column of 256 to 8192 points
+// with P = 512 (256 for N = 256), columns 0 and nlines - 1 in one workgroup as above.
+template <int P, int Q, typename TImg>
+static hipError_t go_xcorr_one(const Stage& s, const StageIO& io, const float2* tw, hipStream_t st) {
+    const int pack = s.real_end_lines && s.nlines >= 2 && env_int("FASTFFT_XCORR_PACK", 1) ? 1 : 0;
+    launch_kernel<k_xcorr_one<P, Q, TImg>>(dim3((unsigned)(s.nlines - pack)), dim3(64 * Q), 0, st,
+            static_cast<const float2*>(io.src), s.im.s1, s.im.es, s.L, static_cast<const TImg*>(io.img), s.gm.s1,
+            static_cast<float2*>(io.dst), s.om.s1, s.om.es, s.M, ((s.o % s.N) + s.N) % s.N, io.scale, tw, s.nlines - 1, pack);
+    return hipGetLastError( );
+}
+
+template <typename TImg>
+static hipError_t try_xcorr_one(const Stage& s, const StageIO& io, const float2* tw, hipStream_t st) {
+    switch ( s.N ) {
+        case 256: return go_xcorr_one<256, 1, TImg>(s, io, tw, st);
+        case 512: return go_xcorr_one<512, 1, TImg>(s, io, tw, st);
+        case 1024: return go_xcorr_one<512, 2, TImg>(s, io, tw, st);
+        case 2048: return go_xcorr_one<512, 4, TImg>(s, io, tw, st);
+        case 4096: return go_xcorr_one<512, 8, TImg>(s, io, tw, st);
+        case 8192: return go_xcorr_one<512, 16, TImg>(s, io, tw, st);
         default: return hipErrorNotSupported;
     }
 }
@@ -139,6 +159,15 @@ hipError_t launch_xcorr(const Stage& s, const StageIO& io, const float2* tw, hip
         if ( ! (io.split_bf16 && io.img_ct == CpxT::c64 && xcorr_toeplitz_covers(s)) )
             return hipErrorNotSupported;
         return go_xcorr_toeplitz(s, io, st);
+    }
+    // one template: columns of the image contiguous (FASTFFT_XCORR_ONE=0 keeps the form that loops
+    // over templates where it applies)
+    if ( ! io.xitems && single_index_lines(s.im) && single_index_lines(s.om) && single_index_lines(s.gm) && s.gm.es == 1 &&
+         s.L <= s.N && s.M >= 1 && s.M <= s.N && s.nlines >= 1 && env_int("FASTFFT_XCORR_ONE", 1) &&
+         ! env_int("FASTFFT_NO_WAVE_XCORR", 0) ) {
+        hipError_t e = io.img_ct == CpxT::c64 ? try_xcorr_one<float2>(s, io, tw, st) : try_xcorr_one<__half2>(s, io, tw, st);
+        if ( e != hipErrorNotSupported )
+            return e;
     }
     // 16-byte image loads: aligned image base (the column starts are checked with the shape)
     const bool col_ok = xcorr_col_covers(s, io.img_ct) && reinterpret_cast<std::uintptr_t>(io.img) % 16 == 0 &&
