@@ -208,6 +208,7 @@ struct fastfft_plan_s {
     // spectrum (sub_fwd); the templates are then correlated on the small frame
     // (sub_xc, window origin 0) with identical results up to rounding.
     bool               sub_active = false;
+    bool               sub_raised = false; // a frame that setup_subframe raised to the kernels' shortest
     int                sub_fx = 0, sub_fy = 0;
     std::vector<Stage> sub_inv, sub_fwd, sub_xc;
     void*              sub_dev = nullptr; // frame (real, FFTW padded), its spectrum, workspace a, b
@@ -278,6 +279,7 @@ static void free_subframe(fastfft_plan p) {
     p->sub_wa     = nullptr;
     p->sub_wb     = nullptr;
     p->sub_active = false;
+    p->sub_raised = false;
     p->sub_inv.clear( );
     p->sub_fwd.clear( );
     p->sub_xc.clear( );
@@ -690,6 +692,14 @@ static fastfft_status setup_batch_kernels(fastfft_plan p, const std::vector<Stag
         if ( best.p > 0 && ! xcorr_col_covers(xcorr_stage_with_p(st[1], best.p), img_ct) )
             best.p = 0;
     }
+    else if ( p->sub_active && (p->sub_raised || p->sub_fy < 512) && ! env_flag("FASTFFT_TUNE") ) {
+        // small frames: no timing at set-up; launches of the whole batch, up to 64 templates, a few
+        // templates per group of columns (24 templates of at most 78^2 in 2048 x 1024: 55 us, 41 of
+        // at most 53^2 in 1024 x 512: 53 us)
+        best.chunk = std::min(n, 64);
+        best.group = n >= 32 ? 4 : n >= 8 ? 2 : 1;
+        how        = "default";
+    }
     else {
         // candidate shapes (the matrix-core pass has one template group per 32 templates)
         const bool       mixed = batch_mixed(p);
@@ -872,22 +882,13 @@ static void column_major_slots(std::vector<Stage>& xc) {
     c.im          = HostLineMap{1, 0, mb, 1};
 }
 
-// Activates the sub-frame form of the batch (see fastfft_plan_s) when the frame
-// is at most a quarter of the plan's, FASTFFT_NO_SUBFRAME is unset and the
-// batched kernels cover the frame's correlation stages; otherwise leaves it off.
-static fastfft_status setup_subframe(fastfft_plan p) {
-    free_subframe(p);
-    const char* off = std::getenv("FASTFFT_NO_SUBFRAME");
-    if ( off && off[0] && std::atoi(off) != 0 )
-        return ok( );
+// Activates the sub-frame form of the batch (see fastfft_plan_s) on an fx by fy frame, at most
+// the plan's size, when the batched kernels cover the frame's correlation stages; otherwise
+// leaves it off.
+static fastfft_status setup_frame(fastfft_plan p, int fx, int fy) {
     const PlanState& st = p->st;
-    const Dims &     in = st.fwd_in, &nn = st.inv_in, &win = st.inv_out;
-    if ( st.transform_dimension != 2 )
-        return ok( );
-    const int fx = next_pow2(in.x + win.x - 1), fy = next_pow2(in.y + win.y - 1);
-    if ( fx >= nn.x || fy >= nn.y || 4L * fx * fy > (long)nn.x * nn.y )
-        return ok( );
-    const int zero[3] = {0, 0, 0};
+    const Dims &     in = st.fwd_in, &nn = st.inv_in;
+    const int        zero[3] = {0, 0, 0};
     // the templates' correlation on the frame: window origin 0 of the frame is lag origin of the plan
     PlanState ps = st;
     ps.fwd_out = ps.inv_in = Dims{fx, fy, 1, 0};
@@ -899,6 +900,8 @@ static fastfft_status setup_subframe(fastfft_plan p) {
     std::vector<Stage> xc, inv, fwd;
     if ( validate(ps).code || build_stages(ps, "xcorr", xc).code || xc.size( ) != 3 )
         return ok( );
+    if ( xc[1].P < 256 && xc[1].N >= 256 ) // the column kernel's shortest sub-transform
+        xc[1] = xcorr_stage_with_p(xc[1], 256);
     // column-major template and output slots, unless FASTFFT_BATCH_ROW_MAJOR=1 (or the
     // column-major row kernels do not cover the frame)
     if ( ! env_flag("FASTFFT_BATCH_ROW_MAJOR") ) {
@@ -918,6 +921,10 @@ static fastfft_status setup_subframe(fastfft_plan p) {
     stages_to_f32(inv);
     stages_to_f32(fwd);
     inv.front( ).src_elem = Elem::cpx_image_type;
+    // the frame starts at the window's first lag, also along an axis it does not shorten (the
+    // planner places windows on trimmed axes only, and so has no origin for a whole one)
+    inv.front( ).o = st.inv_out.y < nn.y ? st.origin[1] : 0;
+    inv.back( ).o  = st.inv_out.x < nn.x ? st.origin[0] : 0;
     for ( const auto* list : {&inv, &fwd, &xc} )
         for ( const Stage& s : *list )
             if ( stage_lds_bytes(s.P) > kMaxLdsBytes )
@@ -948,6 +955,28 @@ static fastfft_status setup_subframe(fastfft_plan p) {
     p->sub_xc     = std::move(xc);
     p->sub_active = true;
     return ok( );
+}
+
+// The sub-frame form where it pays.  First the smallest power-of-two frame, if it is at most a
+// quarter of the plan's.  Where the batched kernels take neither that frame nor the plan's own
+// stages, a batch of four templates or more goes to a frame of at least 512 x 256 points, the
+// shortest those kernels take, up to the plan's size: the alternative is three launches or more
+// per template (24 templates of at most 78^2 in 2048 x 1024: 419 us).  FASTFFT_NO_SUBFRAME
+// leaves both off.
+static fastfft_status setup_subframe(fastfft_plan p, bool plan_covered) {
+    free_subframe(p);
+    if ( env_flag("FASTFFT_NO_SUBFRAME") || p->st.transform_dimension != 2 )
+        return ok( );
+    const Dims &in = p->st.fwd_in, &nn = p->st.inv_in, &win = p->st.inv_out;
+    const int   fx = next_pow2(in.x + win.x - 1), fy = next_pow2(in.y + win.y - 1);
+    if ( fx < nn.x && fy < nn.y && 4L * fx * fy <= (long)nn.x * nn.y )
+        if ( auto rc = setup_frame(p, fx, fy); rc || p->sub_active )
+            return rc;
+    if ( plan_covered || p->batch.size( ) < 4 || nn.x < 512 || nn.y < 256 )
+        return ok( );
+    const fastfft_status rc = setup_frame(p, std::min(std::max(fx, 512), nn.x), std::min(std::max(fy, 256), nn.y));
+    p->sub_raised           = ! rc && p->sub_active;
+    return rc;
 }
 
 // The batch on the sub-frame: image -> frame -> frame spectrum, then every chunk.
@@ -1374,11 +1403,12 @@ fastfft_status fastfft_set_batch(fastfft_plan plan, int n, const void* const* te
         return rc;
     const CpxT img_ct = plan->st.image_type == FASTFFT_IMAGE_C32H ? CpxT::c32h : CpxT::c64;
     fastfft_status rc = ok( );
+    const bool covered = sp->size( ) == 3 && batch_kernels_cover((*sp)[0], (*sp)[1], (*sp)[2], img_ct);
     if ( n > 0 )
-        rc = setup_subframe(plan);
+        rc = setup_subframe(plan, covered);
     if ( ! rc && plan->sub_active )
         rc = setup_batch_kernels(plan, plan->sub_xc, CpxT::c64);
-    else if ( ! rc && n > 0 && sp->size( ) == 3 && batch_kernels_cover((*sp)[0], (*sp)[1], (*sp)[2], img_ct) )
+    else if ( ! rc && n > 0 && covered )
         rc = setup_batch_kernels(plan, *sp, img_ct);
     if ( rc ) {
         plan->batch.clear( );

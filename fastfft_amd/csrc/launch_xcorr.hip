@@ -65,7 +65,7 @@ static hipError_t try_xcorr_col(const Stage& s, const StageIO& io, const float2*
     const int rs = (((s.o / 64) % E) + E) % E;
     auto      by_q = [&](auto qc) -> hipError_t {
         constexpr int Q = decltype(qc)::value;
-        if constexpr ( P * Q > kTwiddleN || (Q == 1 && P != 1024) ) {
+        if constexpr ( P * Q > kTwiddleN ) {
             return hipErrorNotSupported;
         }
         else {
@@ -118,7 +118,7 @@ bool xcorr_col_covers(const Stage& s, CpxT img_ct) {
             s.gm.s1 % per == 0) )
         return false;
     if ( ! (s.P == 256 || s.P == 512 || s.P == 1024) || s.o % 64 != 0 || s.P * s.Q > kTwiddleN || s.P < s.L ||
-         ! ((s.Q == 1 && s.P == 1024) || s.Q == 2 || s.Q == 4 || s.Q == 8 || s.Q == 16) )
+         ! (s.Q == 1 || s.Q == 2 || s.Q == 4 || s.Q == 8 || s.Q == 16) )
         return false;
     const int E  = s.P / 64;
     const int rs = (((s.o / 64) % E) + E) % E;
