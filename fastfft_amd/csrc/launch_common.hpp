@@ -69,15 +69,24 @@ inline int env_int(const char* name, int dflt) {
 }
 
 // Calls f(N, PPW) for the pair-row kernels (pair_rows.hpp): rows of N points, PPW pairs per
-// workgroup, at most FASTFFT_PAIR_GROUP.  Four pairs make 64-byte segments (workgroups of 1024
-// threads at N = 4096; 8192-point rows fit two): 4096^2 forward 71 us with one pair, 56 with
-// two, 56-57 with four; 2730 rows of 4096 points 65, 50 and 45.  Below 64 workgroups' worth of
-// pairs the group is halved to keep CUs busy: 255 rows of 2048 points 16.4, 16.8 and 18.2 us.
+// workgroup, at most FASTFFT_PAIR_GROUP; not supported below min_pairs pairs (rows of 1024 points
+// are taken from one pair on: 128 rows 10.0 us, 10.6 on the row kernels; inverse 10.4 and 12.6).
+// All figures here and at the callers are times of whole 2-D transforms.
+// Four pairs make 64-byte segments (workgroups of 1024 threads at N = 4096; 8192-point rows fit
+// two): 4096^2 forward 67 us with one pair, 55 with two or four; 2730 rows of 4096 points 65, 48
+// and 44.  The group is halved below `groups` workgroups' worth of pairs, which keeps CUs busy.
+// 160, where the rows outweigh the segments (forward, and windows of over half a row): 512 rows of
+// 4096 points 17.7, 18.0 and 21.1 us forward with one, two and four pairs, 17.5, 19.1 and 23.1
+// inverse; 682 rows 25.5, 23.2 and 25.6 forward; 1365 rows 39.0, 31.5 and 29.3.  100 for smaller
+// windows, whose 64-byte reads count for more: 924 rows of 1024 points 18.6, 16.2 and 14.9 us, of
+// 2048 points 26.2, 22.7 and 20.8; 384 rows of 8192 points 25.5 with one pair, 30.4 with two.
 template <class F>
-hipError_t pair_rows_dispatch(int N, int nrows, F&& f) {
+hipError_t pair_rows_dispatch(int N, int nrows, int min_pairs, int groups, F&& f) {
     const int npairs = (nrows + 1) / 2, cap = env_int("FASTFFT_PAIR_GROUP", 4);
+    if ( npairs < env_int("FASTFFT_PAIR_MIN", N == 1024 ? 1 : min_pairs) )
+        return hipErrorNotSupported;
     int       g      = N == 8192 ? 2 : 4;
-    while ( g > 1 && (g > cap || npairs < 64 * g) )
+    while ( g > 1 && (g > cap || npairs < groups * g) )
         g /= 2;
     auto by_n = [&](auto nc) -> hipError_t {
         constexpr int NN = decltype(nc)::value;

@@ -10,20 +10,43 @@
 // The spectrum is stored A[kx][y]: the 2 PPW rows of a workgroup are one 16 PPW-byte
 // segment of every kx, moved 16 bytes per lane; the rows themselves are unit stride.
 // 16 values per thread in registers (T = N / 16 threads per pair), loaded and stored
-// directly, radix-16 Stockham passes, and every exchange moves the real and then the
-// imaginary parts through one LDS buffer of N floats per pair.  That halves the LDS of a
-// pair, and immediate offsets keep the addresses out of the registers (64 at most), so two
-// workgroups of 1024 threads share a CU and one loads or stores while the other computes.
+// directly, and radix-16 Stockham passes.  The exchanges of a workgroup of 1024 threads move the
+// real and then the imaginary parts through one LDS buffer of N floats per pair.  That halves
+// the LDS of a pair, and immediate offsets keep the addresses out of the registers (64 at most),
+// so two such workgroups share a CU and one loads or stores while the other computes.
 // Bound by arithmetic and memory about alike: 4096^2 (134 MB) takes 29.9 us forward and
 // 29.7 us inverse, 4.5 TB/s, where complex exchanges with one workgroup per CU took
 // 38.6 us forward and one row per workgroup with 8-byte gathers 51.7 us inverse.
 #pragma once
+
+#include <type_traits>
 
 #include "rows_wave.hpp"
 
 namespace fastfft_amd {
 
 constexpr int kPairE = 16; // values per thread
+
+// Workgroups of at most 512 threads (8192 points) move whole complex values through LDS: two of
+// them still fit a CU, and half the barriers matter where a launch has few workgroups per CU.
+// 2-D transforms: 2048^2 forward 27.3 -> 26.4 us, inverse 27.0 -> 26.2; 512 rows of 4096 points
+// 17.5 -> 16.9 and 17.5 -> 17.0; 512 rows of 8192 points 30.1 -> 28.6.
+template <int N, int PPW>
+constexpr bool pair_whole = N * PPW <= 8192;
+template <int N, int PPW>
+using PairWord = std::conditional_t<pair_whole<N, PPW>, float2, float>;
+
+// Calls f(part) for every exchange of a pair: the real and the imaginary parts in turn, or whole values.
+template <bool WHOLE, class F>
+__device__ __forceinline__ void for_parts(F&& f) {
+    if constexpr ( ! WHOLE ) {
+        f([](auto& z) -> auto& { return z.x; });
+        f([](auto& z) -> auto& { return z.y; });
+    }
+    else {
+        f([](auto& z) -> auto& { return z; });
+    }
+}
 
 // Exchange slot of element k: one pad word per 16, so that the scatters of the radix-16
 // passes (lane strides 16 and 256) and the unit-stride gathers fall on distinct banks.
@@ -34,7 +57,7 @@ constexpr int                  pair_step(int k) { return k + k / 16; }
 // PPW consecutive pairs start 64 / PPW banks apart, so that the lanes of
 // the segment accesses (PPW pairs, 64 / PPW consecutive k) fall on distinct banks as well.
 template <int N, int PPW>
-constexpr int pair_pitch = N + N / 16 + 64 / PPW;
+constexpr int pair_pitch = N + N / 16 + (pair_whole<N, PPW> ? 32 : 64) / PPW;
 
 // A pair of one wave needs no workgroup barrier in its own exchanges.
 template <int T>
@@ -109,9 +132,9 @@ struct PairTwiddles {
 };
 
 // Stockham passes from stride Ns on: register i of thread t holds element t + T i on entry
-// and on return (natural order).  buf: the pair's N-float exchange buffer.
-template <int N, int Ns, int DIR>
-__device__ __forceinline__ void pair_passes(float2 (&v)[kPairE], float* __restrict__ buf, int t,
+// and on return (natural order).  buf: the pair's exchange buffer of N words.
+template <int N, int PPW, int Ns, int DIR>
+__device__ __forceinline__ void pair_passes(float2 (&v)[kPairE], PairWord<N, PPW>* __restrict__ buf, int t,
                                             const float2* tab, const float2* __restrict__ twm) {
     constexpr int  T = N / kPairE, R = N / Ns < kPairE ? N / Ns : kPairE, B = kPairE / R;
     constexpr bool LAST = Ns * R == N;
@@ -139,12 +162,12 @@ __device__ __forceinline__ void pair_passes(float2 (&v)[kPairE], float* __restri
             v[m + B * r] = u[r];
     }
     if constexpr ( ! LAST ) {
-        auto exchange = [&](auto part) {
+        for_parts<pair_whole<N, PPW>>([&](auto part) {
             pair_sync<T>( ); // the buffer's readers are done
 #pragma unroll
             for ( int m = 0; m < B; m++ ) {
                 const int b = t + T * m, j = b & (Ns - 1);
-                float*    dst = buf + pair_slot((b - j) * R + j); // element (b - j) R + j + r Ns for r < R
+                auto*     dst = buf + pair_slot((b - j) * R + j); // element (b - j) R + j + r Ns for r < R
 #pragma unroll
                 for ( int r = 0; r < R; r++ )
                     dst[Ns == 1 ? r : r * pair_step(Ns)] = part(v[m + B * r]);
@@ -153,10 +176,8 @@ __device__ __forceinline__ void pair_passes(float2 (&v)[kPairE], float* __restri
 #pragma unroll
             for ( int i = 0; i < kPairE; i++ )
                 part(v[i]) = buf[pair_slot(t) + i * pair_step(T)];
-        };
-        exchange([](float2& z) -> float& { return z.x; });
-        exchange([](float2& z) -> float& { return z.y; });
-        pair_passes<N, Ns * R, DIR>(v, buf, t, tab, twm);
+        });
+        pair_passes<N, PPW, Ns * R, DIR>(v, buf, t, tab, twm);
     }
 }
 
@@ -168,14 +189,14 @@ __global__ void __launch_bounds__(N / kPairE * PPW, N / kPairE * PPW == 1024 ? 8
         k_r2c_pair_rows(const TIn* __restrict__ in, LineMap im, int L, float2* __restrict__ out, LineMap om, int nout,
                         int nlines, float pre_scale, const float2* __restrict__ tw) {
     constexpr int T = N / kPairE, NT = T * PPW, H = N / 2, ITER = H / T + 1;
-    __shared__ float  s_x[PPW * pair_pitch<N, PPW>];
-    __shared__ float2 s_tw[kPairTable];
-    PairTable<NT>     table;
+    __shared__ PairWord<N, PPW> s_x[PPW * pair_pitch<N, PPW>];
+    __shared__ float2           s_tw[kPairTable];
+    PairTable<NT>               table;
     table.load(multi_twiddles(tw));
     const int     h     = PPW > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / T) : 0;
     const int     t     = threadIdx.x % T;
     const int     pair0 = xcd_row(blockIdx.x, gridDim.x) * PPW, row = 2 * (pair0 + h);
-    float*        buf   = s_x + h * pair_pitch<N, PPW>;
+    auto*         buf   = s_x + h * pair_pitch<N, PPW>;
     float2        v[kPairE];
     {
         const bool  ha = row < nlines, hb = row + 1 < nlines;
@@ -198,13 +219,14 @@ __global__ void __launch_bounds__(N / kPairE * PPW, N / kPairE * PPW == 1024 ? 8
     }
     table.store(s_tw);
     __syncthreads( );
-    pair_passes<N, 1, -1>(v, buf, t, s_tw, multi_twiddles(tw));
-    // Z in natural order through LDS, real parts first: item (k, g) takes A[k] and B[k] of the
-    // workgroup's pair g, 16 bytes of the segment of k
-    const int    g  = threadIdx.x % PPW, k0 = threadIdx.x / PPW; // k = k0 + T c
-    const float *zk = s_x + g * pair_pitch<N, PPW> + pair_slot(k0), *zn = s_x + g * pair_pitch<N, PPW> + pair_slot(N - k0);
-    float        ax[ITER], by[ITER];
-    auto         spread = [&](auto part) {
+    pair_passes<N, PPW, 1, -1>(v, buf, t, s_tw, multi_twiddles(tw));
+    // Z in natural order through LDS: item (k, g) takes A[k] and B[k] of the workgroup's pair g,
+    // 16 bytes of the segment of k
+    const int   g  = threadIdx.x % PPW, k0 = threadIdx.x / PPW; // k = k0 + T c
+    const auto *zk = s_x + g * pair_pitch<N, PPW> + pair_slot(k0), *zn = s_x + g * pair_pitch<N, PPW> + pair_slot(N - k0);
+    auto*       op = as_global(out) + 2 * pair0;
+    const bool  rows = 2 * (pair0 + g) < nlines;
+    auto        spread = [&](auto part) {
         __syncthreads( );
 #pragma unroll
         for ( int i = 0; i < kPairE; i++ )
@@ -213,24 +235,37 @@ __global__ void __launch_bounds__(N / kPairE * PPW, N / kPairE * PPW == 1024 ? 8
             buf[pair_step(N)] = part(v[0]);
         __syncthreads( );
     };
-    spread([](float2 z) { return z.x; });
-#pragma unroll
-    for ( int c = 0; c < ITER; c++ )
-        if ( c + 1 < ITER || k0 == 0 ) {
-            ax[c] = 0.5f * (zk[c * pair_step(T)] + zn[-c * pair_step(T)]);
-            by[c] = 0.5f * (zn[-c * pair_step(T)] - zk[c * pair_step(T)]);
-        }
-    spread([](float2 z) { return z.y; });
-    auto*      op   = as_global(out) + 2 * pair0;
-    const bool rows = 2 * (pair0 + g) < nlines;
-#pragma unroll
-    for ( int c = 0; c < ITER; c++ ) {
+    // a = (Re A[k], Im A[k]) and b of item c
+    auto store = [&](int c, float2 a, float2 b) {
         const int k = k0 + T * c;
-        if ( k < nout && rows && (c + 1 < ITER || k0 == 0) ) {
-            const float yk = zk[c * pair_step(T)], yn = zn[-c * pair_step(T)];
-            store_cpx_pair(at_bytes(op, 8u * (unsigned)k * (unsigned)om.es + 16u * (unsigned)g), 0,
-                           make_float2(ax[c], 0.5f * (yk - yn)), make_float2(0.5f * (yk + yn), by[c]));
-        }
+        if ( k < nout && rows && (c + 1 < ITER || k0 == 0) )
+            store_cpx_pair(at_bytes(op, 8u * (unsigned)k * (unsigned)om.es + 16u * (unsigned)g), 0, a, b);
+    };
+    if constexpr ( ! pair_whole<N, PPW> ) { // real parts first
+        float ax[ITER], by[ITER];
+        spread([](float2 z) { return z.x; });
+#pragma unroll
+        for ( int c = 0; c < ITER; c++ )
+            if ( c + 1 < ITER || k0 == 0 ) {
+                ax[c] = 0.5f * (zk[c * pair_step(T)] + zn[-c * pair_step(T)]);
+                by[c] = 0.5f * (zn[-c * pair_step(T)] - zk[c * pair_step(T)]);
+            }
+        spread([](float2 z) { return z.y; });
+#pragma unroll
+        for ( int c = 0; c < ITER; c++ )
+            if ( c + 1 < ITER || k0 == 0 ) {
+                const float yk = zk[c * pair_step(T)], yn = zn[-c * pair_step(T)];
+                store(c, make_float2(ax[c], 0.5f * (yk - yn)), make_float2(0.5f * (yk + yn), by[c]));
+            }
+    }
+    else {
+        spread([](float2 z) { return z; });
+#pragma unroll
+        for ( int c = 0; c < ITER; c++ )
+            if ( c + 1 < ITER || k0 == 0 ) {
+                const float2 a = zk[c * pair_step(T)], b = zn[-c * pair_step(T)];
+                store(c, make_float2(0.5f * (a.x + b.x), 0.5f * (a.y - b.y)), make_float2(0.5f * (a.y + b.y), 0.5f * (b.x - a.x)));
+            }
     }
 }
 
@@ -243,14 +278,14 @@ __global__ void __launch_bounds__(N / kPairE * PPW, N / kPairE * PPW == 1024 ? 8
         k_c2r_pair_rows(const float2* __restrict__ in, LineMap im, TOut* __restrict__ out, LineMap om, int M, int o,
                         int nlines, float post_scale, const float2* __restrict__ tw) {
     constexpr int T = N / kPairE, NT = T * PPW, H = N / 2, ITER = H / T + 1;
-    __shared__ float  s_x[PPW * pair_pitch<N, PPW>];
-    __shared__ float2 s_tw[kPairTable];
-    PairTable<NT>     table;
+    __shared__ PairWord<N, PPW> s_x[PPW * pair_pitch<N, PPW>];
+    __shared__ float2           s_tw[kPairTable];
+    PairTable<NT>               table;
     table.load(multi_twiddles(tw));
     const int     h     = PPW > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / T) : 0;
     const int     t     = threadIdx.x % T;
     const int     pair0 = xcd_row(blockIdx.x, gridDim.x) * PPW, row = 2 * (pair0 + h);
-    float*        buf   = s_x + h * pair_pitch<N, PPW>;
+    auto*         buf   = s_x + h * pair_pitch<N, PPW>;
     float2        v[kPairE];
     {
         const auto* ip   = as_global(in) + 2 * pair0;
@@ -271,7 +306,7 @@ __global__ void __launch_bounds__(N / kPairE * PPW, N / kPairE * PPW == 1024 ? 8
             if ( (c == 0 || c + 1 == ITER) && k0 == 0 )
                 u[c].y = u[c].w = 0.f;
         }
-        float *zk = s_x + g * pair_pitch<N, PPW> + pair_slot(k0), *zn = s_x + g * pair_pitch<N, PPW> + pair_slot(N - k0);
+        auto *zk = s_x + g * pair_pitch<N, PPW> + pair_slot(k0), *zn = s_x + g * pair_pitch<N, PPW> + pair_slot(N - k0);
         table.store(s_tw);
         auto   spread = [&](auto lo, auto hi) {
 #pragma unroll
@@ -282,18 +317,26 @@ __global__ void __launch_bounds__(N / kPairE * PPW, N / kPairE * PPW == 1024 ? 8
                 }
             __syncthreads( );
         };
-        spread([](float4 z) { return z.x - z.w; }, [](float4 z) { return z.x + z.w; });
+        auto gather = [&](auto part) {
 #pragma unroll
-        for ( int i = 0; i < kPairE; i++ )
-            v[i].x = buf[pair_slot(t) + i * pair_step(T)];
-        __syncthreads( );
-        spread([](float4 z) { return z.z + z.y; }, [](float4 z) { return z.z - z.y; });
-#pragma unroll
-        for ( int i = 0; i < kPairE; i++ )
-            v[i].y = buf[pair_slot(t) + i * pair_step(T)];
+            for ( int i = 0; i < kPairE; i++ )
+                part(v[i]) = buf[pair_slot(t) + i * pair_step(T)];
+        };
+        if constexpr ( ! pair_whole<N, PPW> ) {
+            spread([](float4 z) { return z.x - z.w; }, [](float4 z) { return z.x + z.w; });
+            gather([](float2& z) -> float& { return z.x; });
+            __syncthreads( );
+            spread([](float4 z) { return z.z + z.y; }, [](float4 z) { return z.z - z.y; });
+            gather([](float2& z) -> float& { return z.y; });
+        }
+        else {
+            spread([](float4 z) { return make_float2(z.x - z.w, z.z + z.y); },
+                   [](float4 z) { return make_float2(z.x + z.w, z.z - z.y); });
+            gather([](float2& z) -> float2& { return z; });
+        }
     }
     __syncthreads( ); // (the first exchange of a one-wave pair orders its own wave only)
-    pair_passes<N, 1, +1>(v, buf, t, s_tw, multi_twiddles(tw));
+    pair_passes<N, PPW, 1, +1>(v, buf, t, s_tw, multi_twiddles(tw));
     if ( row >= nlines )
         return;
     const bool hb = row + 1 < nlines;

@@ -53,3 +53,29 @@ def test_c2r_pair_rows(n, ny, window, origin, dtype):
     got = H.real_window(H.to_host(out).astype(np.float32), *window)
     want = O.inv_2d(spec.astype(np.float32).view(np.complex64).reshape(w, ny), n, ny, *window, *origin, post_scale=post)
     assert O.rel_l2(got, want) < TOLS[dtype]
+
+
+@pytest.mark.parametrize("group", [1, 2, 4])
+@pytest.mark.parametrize("n", [1024, 2048, 4096, 8192])
+def test_pair_rows_of_every_group(monkeypatch, n, group):
+    """Every workgroup shape (whole values or their parts through LDS) at row counts and lengths that the
+    launch rule gives to other shapes or kernels: seven rows are a last pair of one row, and a last
+    workgroup of fewer pairs than its group."""
+    H.log(f"pair rows {n} group {group}")
+    monkeypatch.setenv("FASTFFT_PAIR_MIN", "1")
+    monkeypatch.setenv("FASTFFT_PAIR_GROUP", str(group))
+    rows = 256 * group + 7  # above every rule that halves a group
+    length, ny, window, origin = n - n // 3, 2048, (n // 2 + 5, rows), (n - 9, 3)
+    img = np.random.default_rng(n + group).standard_normal((rows, length)).astype(np.float32)
+    ft = H.make_plan((length, rows, 1), (n, ny, 1), (n, ny, 1), (*window, 1), origin=(*origin, 0))
+    inp = H.to_dev(H.padded_real(img, length).reshape(-1))
+    spec = H.dev_poison(ft.ReturnFwdOutputMemorySize())
+    ft.FwdFFT(inp, spec)
+    got = H.complex_from_f32(H.to_host(spec), (n // 2 + 1, ny))
+    want = O.fwd_2d(H.padded_real(img, length), length, n, ny)
+    assert O.rel_l2(got, want) < TOL
+    out = H.dev_poison(ft.ReturnInvOutputMemorySize())
+    post = 1.0 / (n * ny)
+    ft.InvFFT(spec, out, post_op=H.F.Scale(post))
+    want = O.inv_2d(got, n, ny, *window, *origin, post_scale=post)
+    assert O.rel_l2(H.real_window(H.to_host(out), *window), want) < TOL
