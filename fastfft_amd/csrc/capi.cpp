@@ -193,7 +193,7 @@ struct fastfft_plan_s {
     int           batch_chunk = 0; // 0: per-template launches
     int           batch_group = 0; // templates per template group of the correlation pass (0: the launcher's default)
     int           batch_p     = 0; // sub-transform length of the correlation pass (0: the planner's)
-    std::string   batch_tuned;     // where the launch shape came from: env, cache or timed
+    std::string   batch_tuned;     // where the launch shape came from: env, cache, timed or default (small frames)
     void*         batch_dev   = nullptr;
     RowBatchItem* batch_r2c   = nullptr;
     XcorrItem*    batch_xc    = nullptr;
@@ -209,6 +209,9 @@ struct fastfft_plan_s {
     // (sub_xc, window origin 0) with identical results up to rounding.
     bool               sub_active = false;
     bool               sub_raised = false; // a frame that setup_subframe raised to the kernels' shortest
+    // A small frame (raised, or of lags and templates under 256 along y) is a faster way to the same
+    // FP32 maps only: precision, statistics and stage timing answer as for the plan's own stages.
+    bool               sub_small = false, plan_batched = false; // plan_batched: the batched kernels take those
     int                sub_fx = 0, sub_fy = 0;
     std::vector<Stage> sub_inv, sub_fwd, sub_xc;
     void*              sub_dev = nullptr; // frame (real, FFTW padded), its spectrum, workspace a, b
@@ -280,6 +283,7 @@ static void free_subframe(fastfft_plan p) {
     p->sub_wb     = nullptr;
     p->sub_active = false;
     p->sub_raised = false;
+    p->sub_small  = false;
     p->sub_inv.clear( );
     p->sub_fwd.clear( );
     p->sub_xc.clear( );
@@ -631,7 +635,7 @@ static int next_pow2(int v);
 // its R2C x-pass, whose output (the frame in mixed form, with the frame spectrum's column
 // layout) the matrix-core correlation pass reads in place of the spectrum.
 static bool batch_mixed(fastfft_plan p) {
-    if ( ! p->sub_active || p->precision != FASTFFT_PRECISION_SPLIT_BF16 || p->sub_fwd.size( ) != 2 ||
+    if ( ! p->sub_active || p->sub_small || p->precision != FASTFFT_PRECISION_SPLIT_BF16 || p->sub_fwd.size( ) != 2 ||
          p->sub_xc.size( ) != 3 )
         return false;
     const Stage &f = p->sub_fwd[0], &x = p->sub_xc[1];
@@ -887,7 +891,7 @@ static void column_major_slots(std::vector<Stage>& xc) {
 // leaves it off.
 static fastfft_status setup_frame(fastfft_plan p, int fx, int fy) {
     const PlanState& st = p->st;
-    const Dims &     in = st.fwd_in, &nn = st.inv_in;
+    const Dims &     nn = st.inv_in;
     const int        zero[3] = {0, 0, 0};
     // the templates' correlation on the frame: window origin 0 of the frame is lag origin of the plan
     PlanState ps = st;
@@ -900,7 +904,8 @@ static fastfft_status setup_frame(fastfft_plan p, int fx, int fy) {
     std::vector<Stage> xc, inv, fwd;
     if ( validate(ps).code || build_stages(ps, "xcorr", xc).code || xc.size( ) != 3 )
         return ok( );
-    if ( xc[1].P < 256 && xc[1].N >= 256 ) // the column kernel's shortest sub-transform
+    const bool lifted = xc[1].P < 256 && xc[1].N >= 256;
+    if ( lifted ) // the column kernel's shortest sub-transform
         xc[1] = xcorr_stage_with_p(xc[1], 256);
     // column-major template and output slots, unless FASTFFT_BATCH_ROW_MAJOR=1 (or the
     // column-major row kernels do not cover the frame)
@@ -942,6 +947,10 @@ static fastfft_status setup_frame(fastfft_plan p, int fx, int fy) {
     hipError_t   e     = dev_alloc(&p->sub_dev, bytes);
     if ( e != hipSuccess ) {
         p->sub_dev = nullptr;
+        if ( lifted ) { // (a batch that can do without)
+            (void)hipGetLastError( );
+            return ok( );
+        }
         return hip_fail(e, "hipMalloc(batch frame)");
     }
     p->sub_s      = static_cast<float*>(p->sub_dev);
@@ -953,6 +962,7 @@ static fastfft_status setup_frame(fastfft_plan p, int fx, int fy) {
     p->sub_inv    = std::move(inv);
     p->sub_fwd    = std::move(fwd);
     p->sub_xc     = std::move(xc);
+    p->sub_small  = lifted;
     p->sub_active = true;
     return ok( );
 }
@@ -974,9 +984,10 @@ static fastfft_status setup_subframe(fastfft_plan p, bool plan_covered) {
             return rc;
     if ( plan_covered || p->batch.size( ) < 4 || nn.x < 512 || nn.y < 256 )
         return ok( );
-    const fastfft_status rc = setup_frame(p, std::min(std::max(fx, 512), nn.x), std::min(std::max(fy, 256), nn.y));
-    p->sub_raised           = ! rc && p->sub_active;
-    return rc;
+    if ( setup_frame(p, std::min(std::max(fx, 512), nn.x), std::min(std::max(fy, 256), nn.y)) )
+        (void)hipGetLastError( ); // no memory for it: the batch does without
+    p->sub_raised = p->sub_small = p->sub_active;
+    return ok( );
 }
 
 // The batch on the sub-frame: image -> frame -> frame spectrum, then every chunk.
@@ -1404,11 +1415,17 @@ fastfft_status fastfft_set_batch(fastfft_plan plan, int n, const void* const* te
     const CpxT img_ct = plan->st.image_type == FASTFFT_IMAGE_C32H ? CpxT::c32h : CpxT::c64;
     fastfft_status rc = ok( );
     const bool covered = sp->size( ) == 3 && batch_kernels_cover((*sp)[0], (*sp)[1], (*sp)[2], img_ct);
+    plan->plan_batched = covered;
     if ( n > 0 )
         rc = setup_subframe(plan, covered);
     if ( ! rc && plan->sub_active )
         rc = setup_batch_kernels(plan, plan->sub_xc, CpxT::c64);
-    else if ( ! rc && n > 0 && covered )
+    if ( plan->sub_small && rc ) { // no memory for a small frame: the batch does without
+        free_batch_device(plan);
+        free_subframe(plan);
+        rc = ok( );
+    }
+    if ( ! rc && n > 0 && covered && ! plan->sub_active )
         rc = setup_batch_kernels(plan, *sp, img_ct);
     if ( rc ) {
         plan->batch.clear( );
@@ -1495,7 +1512,8 @@ fastfft_status fastfft_run_batch_stage(fastfft_plan plan, int stage, const void*
         return rc;
     if ( stage < 0 || stage > 4 || ! image_to_search )
         return fail(FASTFFT_INVALID_ARGUMENT, "run_batch_stage: stage must be 0..4 and the image not null");
-    if ( plan->batch_chunk <= 0 || reinterpret_cast<std::uintptr_t>(image_to_search) % 16 != 0 )
+    if ( plan->batch_chunk <= 0 || (plan->sub_small && ! plan->plan_batched) ||
+         reinterpret_cast<std::uintptr_t>(image_to_search) % 16 != 0 )
         return fail(FASTFFT_UNSUPPORTED, "run_batch_stage: the batch runs per template (no batched kernels)");
     const std::vector<Stage>* sp = nullptr;
     if ( auto rc = get_stages(plan, 2, &sp) )
@@ -1656,7 +1674,7 @@ fastfft_status fastfft_run_stages(fastfft_plan plan, const char* op, int first, 
 
 // the C2R stage of the batch's active form (frame or full)
 static fastfft_status batch_c2r_stage(fastfft_plan p, const Stage** out) {
-    if ( p->batch.empty( ) || p->batch_chunk <= 0 )
+    if ( p->batch.empty( ) || p->batch_chunk <= 0 || (p->sub_small && ! p->plan_batched) )
         return fail(FASTFFT_UNSUPPORTED, "batch statistics need a batch set on the batched kernels (fastfft_set_batch)");
     if ( p->sub_active ) {
         *out = &p->sub_xc[2];
@@ -1684,9 +1702,13 @@ fastfft_status fastfft_set_batch_stats(fastfft_plan plan, float* mip, int* best,
     const Stage* c2r = nullptr;
     if ( auto rc = batch_c2r_stage(plan, &c2r) )
         return rc;
-    if ( ! c2r_stats_covers(*c2r) )
+    const std::vector<Stage>* own = nullptr;
+    if ( plan->sub_small )
+        if ( auto rc = get_stages(plan, 2, &own) )
+            return rc;
+    if ( const Stage* asked = own ? &own->back( ) : c2r; ! c2r_stats_covers(*c2r) || ! c2r_stats_covers(*asked) )
         return fail(FASTFFT_UNSUPPORTED, "set_batch_stats: the statistics form covers 512- and 1024-point frames along x "
-                                         "(this batch runs " + std::to_string(c2r->N) + "-point rows)");
+                                         "(this batch runs " + std::to_string(asked->N) + "-point rows)");
     // partial maps of the template groups, allocated once per batch (calls allocate nothing)
     float* part = plan->batch_stats.part;
     if ( ! part ) {

@@ -1,10 +1,11 @@
 // Fused correlation pass of FwdImageInvFFT.
 //
-// Lines of a single index (the 2-D second axis) with P in {256, 512, 1024}, a
-// window origin that is a multiple of 64 placed at register rotation 0 or E/2,
-// N = P*Q <= 8192 and a contiguous, 16-byte aligned image column run the
-// workgroup-per-column kernel of xcorr_col.hpp; every other shape runs the
-// generic line kernel.
+// Lines of a single index (the 2-D second axis) with a contiguous image column: one template
+// of any length L <= N, window and origin runs the workgroup-per-column kernel of
+// xcorr_one.hpp (N = 256 .. 8192), several templates the loop form of xcorr_col.hpp (P in {256,
+// 512, 1024}, a window origin that is a multiple of 64 placed at register rotation 0 or E/2,
+// N = P*Q <= 8192, 16-byte aligned image columns).  Strided lines of 64 to 512 points (the
+// 3-D z-pass) run lines.hpp, every other shape the generic line kernel.
 #include <algorithm>
 #include <cstdint>
 

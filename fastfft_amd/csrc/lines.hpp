@@ -4,8 +4,8 @@
 // include/detail/memory_addressing.h:25-104) and the 256- and 512-point passes of the
 // 2-D ones.
 //
-// T = N / 16 threads per line, 16 values per thread (thread t holds elements t + T i),
-// radix-16 Stockham passes: one LDS exchange up to 256 points, two at 512.
+// T = N / E threads per line, E = 16 or 8 values per thread (line_values; thread t holds
+// elements t + T i), radix-E Stockham passes: at most two LDS exchanges.
 //   IN_X / OUT_X: the lines lie next to each other and their elements far apart (a
 //     z-pass, the transposed side of an x-pass): consecutive lanes take consecutive
 //     lines, so that the 16 lines of a workgroup are one 128-byte segment per element,
@@ -27,7 +27,7 @@
 
 namespace fastfft_amd {
 
-// Values per thread: 16 up to 128 points; 8 at 512 (16 needs a radix-2 pass after the same two
+// Values per thread: 16 at 128 points; 8 at 64 (twice the threads of short lines), at 512 (16 needs a radix-2 pass after the same two
 // exchanges: 512-point passes of 512^3 143 + 48 us against 118 + 42) and at 256 points, where
 // twice the waves outweigh the second exchange (fused z-pass of 256^3 35.3 us with 16, 30.4
 // with 8; C2R rows 9.6 and 8.6) except for real rows (6.9 and 8.7 us for 5,084 of them).
@@ -157,18 +157,17 @@ __device__ __forceinline__ void line_passes(float2 (&v)[E], float2* bw, int tw, 
 // single-index one) are cut into tiles of LT, the last one partly filled.
 struct LineTile {
     int line0, count; // first line, lines that exist
-    __device__ __forceinline__ LineTile(int tile, int per, int nlines, int lt) {
+    __device__ __forceinline__ LineTile(int tile, int per, int lt) {
         const int tpg = (per + lt - 1) / lt, g = tile / tpg, y0 = (tile - g * tpg) * lt;
         line0 = g * per + y0;
         count = min(lt, per - y0);
-        (void)nlines;
     }
 };
 
 // element-index step between neighbouring lines of a tile
 __device__ __forceinline__ unsigned line_stride(const LineMap& m) { return (unsigned)(m.n2 > 1 ? m.s2 : m.s1); }
 
-// Grid: groups x ceil(per / lines) workgroups of lines_per_workgroup * N / 16 threads
+// Grid: groups x ceil(per / LT) workgroups of LT N / line_values threads
 // (HERM: two rows per transform).  flags bit 0: workgroups in XCD-contiguous ranges.
 template <int N, int LT, int DIR, typename TIn, bool HERM, typename TOut, bool IN_X, bool OUT_X>
 __global__ void __launch_bounds__(LT* N / line_values(N, is_real_element<TIn>))
@@ -183,7 +182,7 @@ __global__ void __launch_bounds__(LT* N / line_values(N, is_real_element<TIn>))
     __shared__ float2 s_tw[line_table_size<N, E>( )];
     LineTable<N, E, LT * T> table;
     table.load(multi_twiddles(tw));
-    const LineTile    tile((flags & 1) ? xcd_row(blockIdx.x, gridDim.x) : (int)blockIdx.x, im.n2 > 1 ? im.n2 : nlines, nlines,
+    const LineTile    tile((flags & 1) ? xcd_row(blockIdx.x, gridDim.x) : (int)blockIdx.x, im.n2 > 1 ? im.n2 : nlines,
                            LT * ROWS);
     const int         li = IN_X ? threadIdx.x % LT : threadIdx.x / T, ti = IN_X ? threadIdx.x / LT : threadIdx.x % T;
     const int         lo = OUT_X ? threadIdx.x % LT : threadIdx.x / T, to = OUT_X ? threadIdx.x / LT : threadIdx.x % T;
@@ -266,7 +265,7 @@ __global__ void __launch_bounds__(kTileLines* N / line_values(N, false))
     __shared__ float2 s_tw[line_table_size<N, E>( )];
     LineTable<N, E, LT * T> table;
     table.load(multi_twiddles(tw));
-    const LineTile    tile(blockIdx.x, nlines, nlines, LT);
+    const LineTile    tile(blockIdx.x, nlines, LT);
     const int         l = threadIdx.x % LT, t = threadIdx.x / LT;
     const bool        mine = l < tile.count;
     float2*           buf  = s_x + l * line_pitch<N, E>;

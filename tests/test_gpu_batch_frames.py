@@ -54,3 +54,20 @@ def test_small_template_batch(sizes, n, nout, origin, frame, dtype):
         gx, gy, gv = O.argmax_2d(got)
         px, py = (int(v) for v in H.to_host(peaks)[2 * i: 2 * i + 2])
         assert (px, py) == (gx, gy) and abs(float(H.to_host(vals)[i]) - gv) <= 1e-6 * abs(gv)
+
+
+def test_small_frame_answers_as_the_plan():
+    """A frame that only these small templates get leaves what the plan's own stages answer: no statistics or
+    stage timing where those have no batched kernels, and FP32 whatever the precision asked for."""
+    n, nout, size, count = (2048, 1024), (500, 500), (300, 300), 4
+    ft = H.make_plan((*size, 1), (*n, 1), (*n, 1), (*nout, 1), origin=(-250, -250, 0))
+    rng = np.random.default_rng(5)
+    bufs = [H.to_dev(H.padded_real(rng.standard_normal(size[::-1]).astype(np.float32), size[0]).reshape(-1)) for _ in range(count)]
+    outs = [H.dev_poison(ft.ReturnInvOutputMemorySize()) for _ in range(count)]
+    ft.SetPrecision("split_bf16")
+    ft.SetBatch(bufs, [size] * count, outs)
+    line = ft.Describe("batch").splitlines()[0]
+    assert "frame=1024x1024" in line and "precision=fp32" in line
+    maps = [torch.zeros(nout[0] * nout[1], dtype=t, device="cuda:0") for t in (torch.float32, torch.int32, torch.float32, torch.float32)]
+    with pytest.raises(H.F.FastFFTError, match="UNSUPPORTED"):
+        ft.SetBatchStats(*maps)
