@@ -233,7 +233,7 @@ static hipError_t go_pair_rows(const Stage& s, const StageIO& io, const float2* 
 }
 
 static hipError_t try_pair_rows(const Stage& s, const StageIO& io, const float2* tw, hipStream_t st) {
-    if ( s.kind != StageKind::fwd_real || ! io.src_real || io.dst_real || io.dst_ct != CpxT::c64 || s.nlines < 1 ||
+    if ( s.N < 1024 || s.kind != StageKind::fwd_real || ! io.src_real || io.dst_real || io.dst_ct != CpxT::c64 || s.nlines < 1 ||
          s.L > s.N || s.nout < 1 || s.nout > s.N / 2 + 1 || s.im.n2 != 1 || s.im.es != 1 || s.om.n2 != 1 || s.om.s1 != 1 ||
          s.om.es % 2 != 0 || s.om.es < s.nlines ||
          reinterpret_cast<std::uintptr_t>(io.dst) % 16 != 0 || env_int("FASTFFT_NO_PAIR_LINES", 0) )

@@ -493,7 +493,7 @@ static hipError_t go_c2r_pair_rows(const Stage& s, const StageIO& io, const floa
 }
 
 static hipError_t try_c2r_pair_rows(const Stage& s, const StageIO& io, const float2* tw, hipStream_t st) {
-    if ( s.kind != StageKind::inv_c2r || io.amax || io.src_real || io.src_ct != CpxT::c64 || ! io.dst_real || s.nlines < 1 ||
+    if ( s.N < 1024 || s.kind != StageKind::inv_c2r || io.amax || io.src_real || io.src_ct != CpxT::c64 || ! io.dst_real || s.nlines < 1 ||
          s.M < 1 || s.M > s.N || s.im.n2 != 1 || s.im.s1 != 1 || s.im.es % 2 != 0 || s.im.es < s.nlines ||
          s.om.n2 != 1 || s.om.es != 1 || reinterpret_cast<std::uintptr_t>(io.src) % 16 != 0 ||
          env_int("FASTFFT_NO_PAIR_LINES", 0) || env_int("FASTFFT_NO_FULL_LINES", 0) )

@@ -64,7 +64,7 @@ bool lines_cover(const Stage& s) {
 }
 
 hipError_t launch_lines(const Stage& s, const StageIO& io, const float2* tw, hipStream_t st) {
-    if ( env_int("FASTFFT_NO_TILE_LINES", 0) || ! lines_cover(s) )
+    if ( ! lines_cover(s) || env_int("FASTFFT_NO_TILE_LINES", 0) )
         return hipErrorNotSupported;
     const bool r2c = s.kind == StageKind::fwd_real;
     const bool fwd = s.kind == StageKind::fwd_cpx || r2c, c2r = s.kind == StageKind::inv_c2r;
