@@ -85,6 +85,7 @@ void log_launch(const char* tag, dim3 grid, dim3 block, size_t lds) {
 namespace {
 
 thread_local std::string g_last_error;
+thread_local hipError_t  g_last_hip = hipSuccess; // of the last hip_fail
 
 fastfft_status fail(int code, const std::string& msg) {
     g_last_error = msg;
@@ -94,7 +95,17 @@ fastfft_status fail(int code, const std::string& msg) {
 fastfft_status ok( ) { return FASTFFT_SUCCESS; }
 
 fastfft_status hip_fail(hipError_t e, const char* what) {
+    g_last_hip = e;
     return fail(FASTFFT_HIP_ERROR, std::string(what) + ": " + hipGetErrorString(e));
+}
+
+// Takes back a failure for want of device memory, where the call can do without what it asked for: the runtime's
+// thread error is cleared, which the next launch would otherwise report as its own.  False: another failure.
+bool forgive_no_memory(fastfft_status rc) {
+    if ( rc != FASTFFT_OUT_OF_MEMORY && ! (rc == FASTFFT_HIP_ERROR && g_last_hip == hipErrorOutOfMemory) )
+        return false;
+    (void)hipGetLastError( );
+    return true;
 }
 
 // Device allocation of a plan's internal buffers (workspace, argmax scratch,
@@ -947,11 +958,8 @@ static fastfft_status setup_frame(fastfft_plan p, int fx, int fy) {
     hipError_t   e     = dev_alloc(&p->sub_dev, bytes);
     if ( e != hipSuccess ) {
         p->sub_dev = nullptr;
-        if ( lifted ) { // (a batch that can do without)
-            (void)hipGetLastError( );
-            return ok( );
-        }
-        return hip_fail(e, "hipMalloc(batch frame)");
+        const fastfft_status rc = hip_fail(e, "hipMalloc(batch frame)");
+        return lifted && forgive_no_memory(rc) ? ok( ) : rc; // (a batch that can do without)
     }
     p->sub_s      = static_cast<float*>(p->sub_dev);
     p->sub_h      = reinterpret_cast<float2*>(p->sub_s + s_floats);
@@ -984,8 +992,9 @@ static fastfft_status setup_subframe(fastfft_plan p, bool plan_covered) {
             return rc;
     if ( plan_covered || p->batch.size( ) < 4 || nn.x < 512 || nn.y < 256 )
         return ok( );
-    if ( setup_frame(p, std::min(std::max(fx, 512), nn.x), std::min(std::max(fy, 256), nn.y)) )
-        (void)hipGetLastError( ); // no memory for it: the batch does without
+    if ( auto rc = setup_frame(p, std::min(std::max(fx, 512), nn.x), std::min(std::max(fy, 256), nn.y));
+         rc && ! forgive_no_memory(rc) )
+        return rc;
     p->sub_raised = p->sub_small = p->sub_active;
     return ok( );
 }
@@ -1420,7 +1429,7 @@ fastfft_status fastfft_set_batch(fastfft_plan plan, int n, const void* const* te
         rc = setup_subframe(plan, covered);
     if ( ! rc && plan->sub_active )
         rc = setup_batch_kernels(plan, plan->sub_xc, CpxT::c64);
-    if ( plan->sub_small && rc ) { // no memory for a small frame: the batch does without
+    if ( rc && plan->sub_small && forgive_no_memory(rc) ) { // no memory for a small frame: the batch does without
         free_batch_device(plan);
         free_subframe(plan);
         rc = ok( );
