@@ -220,9 +220,12 @@ struct fastfft_plan_s {
     // (sub_xc, window origin 0) with identical results up to rounding.
     bool               sub_active = false;
     bool               sub_raised = false; // a frame that setup_subframe raised to the kernels' shortest
-    // A small frame (raised, or of lags and templates under 256 along y) is a faster way to the same
-    // FP32 maps only: precision, statistics and stage timing answer as for the plan's own stages.
-    bool               sub_small = false, plan_batched = false; // plan_batched: the batched kernels take those
+    // Stages with short columns (one sub-transform of under 1024 points) and raised frames are a faster way to
+    // the same FP32 maps only: precision, statistics and stage timing answer as for the plan's own stages, where
+    // those columns are not short and the batched kernels take them (plan_batched), else as per template.
+    bool               sub_small = false;   // the frame is such a form
+    bool               batch_small = false; // the batch's active form (frame or the plan's own stages) is one
+    bool               plan_batched = false;
     int                sub_fx = 0, sub_fy = 0;
     std::vector<Stage> sub_inv, sub_fwd, sub_xc;
     void*              sub_dev = nullptr; // frame (real, FFTW padded), its spectrum, workspace a, b
@@ -281,6 +284,7 @@ static void free_batch_device(fastfft_plan p) {
     p->batch_chunk = 0;
     p->batch_group = 0;
     p->batch_p     = 0;
+    p->batch_small = false;
     p->batch_tuned.clear( );
 }
 
@@ -897,9 +901,14 @@ static void column_major_slots(std::vector<Stage>& xc) {
     c.im          = HostLineMap{1, 0, mb, 1};
 }
 
+// Columns of one sub-transform of under 1024 points: what the batched kernels take of them, they
+// take for speed alone (see fastfft_plan_s).
+static bool short_columns(const Stage& xcorr) { return xcorr.Q == 1 && xcorr.P < 1024; }
+
 // Activates the sub-frame form of the batch (see fastfft_plan_s) on an fx by fy frame, at most
 // the plan's size, when the batched kernels cover the frame's correlation stages; otherwise
-// leaves it off.
+// leaves it off.  One template does not pay for the reduction of the image to a frame of short
+// columns (300^2 to 200^2 lags of a 1024^2 image: 34.4 us on a frame of 512^2, 19.6 on the plan's own stages).
 static fastfft_status setup_frame(fastfft_plan p, int fx, int fy) {
     const PlanState& st = p->st;
     const Dims &     nn = st.inv_in;
@@ -915,8 +924,7 @@ static fastfft_status setup_frame(fastfft_plan p, int fx, int fy) {
     std::vector<Stage> xc, inv, fwd;
     if ( validate(ps).code || build_stages(ps, "xcorr", xc).code || xc.size( ) != 3 )
         return ok( );
-    const bool lifted = xc[1].P < 256 && xc[1].N >= 256;
-    if ( lifted ) // the column kernel's shortest sub-transform
+    if ( xc[1].P < 256 && xc[1].N >= 256 ) // the column kernel's shortest sub-transform
         xc[1] = xcorr_stage_with_p(xc[1], 256);
     // column-major template and output slots, unless FASTFFT_BATCH_ROW_MAJOR=1 (or the
     // column-major row kernels do not cover the frame)
@@ -926,7 +934,8 @@ static fastfft_status setup_frame(fastfft_plan p, int fx, int fy) {
         if ( batch_kernels_cover(cm[0], cm[1], cm[2], CpxT::c64) )
             xc = std::move(cm);
     }
-    if ( ! batch_kernels_cover(xc[0], xc[1], xc[2], CpxT::c64) )
+    const bool small = short_columns(xc[1]);
+    if ( ! batch_kernels_cover(xc[0], xc[1], xc[2], CpxT::c64) || (small && p->batch.size( ) < 2) )
         return ok( );
     // the image reduced to the frame: trimmed inverse of the N-frame spectrum (read in the plan's image type) ...
     PlanState pi = frame_plan(FASTFFT_INPUT_F32, nn, Dims{fx, fy, 1, 0}, st.origin);
@@ -959,7 +968,7 @@ static fastfft_status setup_frame(fastfft_plan p, int fx, int fy) {
     if ( e != hipSuccess ) {
         p->sub_dev = nullptr;
         const fastfft_status rc = hip_fail(e, "hipMalloc(batch frame)");
-        return lifted && forgive_no_memory(rc) ? ok( ) : rc; // (a batch that can do without)
+        return small && forgive_no_memory(rc) ? ok( ) : rc; // (a batch that can do without)
     }
     p->sub_s      = static_cast<float*>(p->sub_dev);
     p->sub_h      = reinterpret_cast<float2*>(p->sub_s + s_floats);
@@ -970,7 +979,7 @@ static fastfft_status setup_frame(fastfft_plan p, int fx, int fy) {
     p->sub_inv    = std::move(inv);
     p->sub_fwd    = std::move(fwd);
     p->sub_xc     = std::move(xc);
-    p->sub_small  = lifted;
+    p->sub_small  = small;
     p->sub_active = true;
     return ok( );
 }
@@ -1424,7 +1433,8 @@ fastfft_status fastfft_set_batch(fastfft_plan plan, int n, const void* const* te
     const CpxT img_ct = plan->st.image_type == FASTFFT_IMAGE_C32H ? CpxT::c32h : CpxT::c64;
     fastfft_status rc = ok( );
     const bool covered = sp->size( ) == 3 && batch_kernels_cover((*sp)[0], (*sp)[1], (*sp)[2], img_ct);
-    plan->plan_batched = covered;
+    const bool own_short = covered && short_columns((*sp)[1]);
+    plan->plan_batched   = covered && ! own_short;
     if ( n > 0 )
         rc = setup_subframe(plan, covered);
     if ( ! rc && plan->sub_active )
@@ -1434,8 +1444,14 @@ fastfft_status fastfft_set_batch(fastfft_plan plan, int n, const void* const* te
         free_subframe(plan);
         rc = ok( );
     }
-    if ( ! rc && n > 0 && covered && ! plan->sub_active )
+    if ( ! rc && n > 0 && covered && ! plan->sub_active ) {
         rc = setup_batch_kernels(plan, *sp, img_ct);
+        if ( rc && own_short && forgive_no_memory(rc) ) { // likewise
+            free_batch_device(plan);
+            rc = ok( );
+        }
+    }
+    plan->batch_small = plan->sub_active ? plan->sub_small : own_short;
     if ( rc ) {
         plan->batch.clear( );
         plan->batch_stages.clear( );
@@ -1521,7 +1537,7 @@ fastfft_status fastfft_run_batch_stage(fastfft_plan plan, int stage, const void*
         return rc;
     if ( stage < 0 || stage > 4 || ! image_to_search )
         return fail(FASTFFT_INVALID_ARGUMENT, "run_batch_stage: stage must be 0..4 and the image not null");
-    if ( plan->batch_chunk <= 0 || (plan->sub_small && ! plan->plan_batched) ||
+    if ( plan->batch_chunk <= 0 || (plan->batch_small && ! plan->plan_batched) ||
          reinterpret_cast<std::uintptr_t>(image_to_search) % 16 != 0 )
         return fail(FASTFFT_UNSUPPORTED, "run_batch_stage: the batch runs per template (no batched kernels)");
     const std::vector<Stage>* sp = nullptr;
@@ -1683,7 +1699,7 @@ fastfft_status fastfft_run_stages(fastfft_plan plan, const char* op, int first, 
 
 // the C2R stage of the batch's active form (frame or full)
 static fastfft_status batch_c2r_stage(fastfft_plan p, const Stage** out) {
-    if ( p->batch.empty( ) || p->batch_chunk <= 0 || (p->sub_small && ! p->plan_batched) )
+    if ( p->batch.empty( ) || p->batch_chunk <= 0 || (p->batch_small && ! p->plan_batched) )
         return fail(FASTFFT_UNSUPPORTED, "batch statistics need a batch set on the batched kernels (fastfft_set_batch)");
     if ( p->sub_active ) {
         *out = &p->sub_xc[2];
@@ -1712,7 +1728,7 @@ fastfft_status fastfft_set_batch_stats(fastfft_plan plan, float* mip, int* best,
     if ( auto rc = batch_c2r_stage(plan, &c2r) )
         return rc;
     const std::vector<Stage>* own = nullptr;
-    if ( plan->sub_small )
+    if ( plan->batch_small )
         if ( auto rc = get_stages(plan, 2, &own) )
             return rc;
     if ( const Stage* asked = own ? &own->back( ) : c2r; ! c2r_stats_covers(*c2r) || ! c2r_stats_covers(*asked) )
