@@ -909,7 +909,8 @@ static bool short_columns(const Stage& xcorr) { return xcorr.Q == 1 && xcorr.P <
 // the plan's size, when the batched kernels cover the frame's correlation stages; otherwise
 // leaves it off.  One template does not pay for the reduction of the image to a frame of short
 // columns (300^2 to 200^2 lags of a 1024^2 image: 34.4 us on a frame of 512^2, 19.6 on the plan's own stages).
-static fastfft_status setup_frame(fastfft_plan p, int fx, int fy) {
+// capturing: the plan's stream is being captured, and a batch that could do without a frame allocates none.
+static fastfft_status setup_frame(fastfft_plan p, int fx, int fy, bool capturing) {
     const PlanState& st = p->st;
     const Dims &     nn = st.inv_in;
     const int        zero[3] = {0, 0, 0};
@@ -935,7 +936,7 @@ static fastfft_status setup_frame(fastfft_plan p, int fx, int fy) {
             xc = std::move(cm);
     }
     const bool small = short_columns(xc[1]);
-    if ( ! batch_kernels_cover(xc[0], xc[1], xc[2], CpxT::c64) || (small && p->batch.size( ) < 2) )
+    if ( ! batch_kernels_cover(xc[0], xc[1], xc[2], CpxT::c64) || (small && (p->batch.size( ) < 2 || capturing)) )
         return ok( );
     // the image reduced to the frame: trimmed inverse of the N-frame spectrum (read in the plan's image type) ...
     PlanState pi = frame_plan(FASTFFT_INPUT_F32, nn, Dims{fx, fy, 1, 0}, st.origin);
@@ -990,18 +991,18 @@ static fastfft_status setup_frame(fastfft_plan p, int fx, int fy) {
 // shortest those kernels take, up to the plan's size: the alternative is three launches or more
 // per template (24 templates of at most 78^2 in 2048 x 1024: 419 us).  FASTFFT_NO_SUBFRAME
 // leaves both off.
-static fastfft_status setup_subframe(fastfft_plan p, bool plan_covered) {
+static fastfft_status setup_subframe(fastfft_plan p, bool plan_covered, bool capturing) {
     free_subframe(p);
     if ( env_flag("FASTFFT_NO_SUBFRAME") || p->st.transform_dimension != 2 )
         return ok( );
     const Dims &in = p->st.fwd_in, &nn = p->st.inv_in, &win = p->st.inv_out;
     const int   fx = next_pow2(in.x + win.x - 1), fy = next_pow2(in.y + win.y - 1);
     if ( fx < nn.x && fy < nn.y && 4L * fx * fy <= (long)nn.x * nn.y )
-        if ( auto rc = setup_frame(p, fx, fy); rc || p->sub_active )
+        if ( auto rc = setup_frame(p, fx, fy, capturing); rc || p->sub_active )
             return rc;
-    if ( plan_covered || p->batch.size( ) < 4 || nn.x < 512 || nn.y < 256 )
+    if ( plan_covered || capturing || p->batch.size( ) < 4 || nn.x < 512 || nn.y < 256 )
         return ok( );
-    if ( auto rc = setup_frame(p, std::min(std::max(fx, 512), nn.x), std::min(std::max(fy, 256), nn.y));
+    if ( auto rc = setup_frame(p, std::min(std::max(fx, 512), nn.x), std::min(std::max(fy, 256), nn.y), capturing);
          rc && ! forgive_no_memory(rc) )
         return rc;
     p->sub_raised = p->sub_small = p->sub_active;
@@ -1432,11 +1433,17 @@ fastfft_status fastfft_set_batch(fastfft_plan plan, int n, const void* const* te
         return rc;
     const CpxT img_ct = plan->st.image_type == FASTFFT_IMAGE_C32H ? CpxT::c32h : CpxT::c64;
     fastfft_status rc = ok( );
-    const bool covered = sp->size( ) == 3 && batch_kernels_cover((*sp)[0], (*sp)[1], (*sp)[2], img_ct);
+    // (allocation during a capture would invalidate it)
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if ( n > 0 && hipStreamIsCapturing(plan->stream, &cs) != hipSuccess )
+        (void)hipGetLastError( ); // (asked only: nothing failed)
+    const bool capturing = cs != hipStreamCaptureStatusNone;
+    bool       covered   = sp->size( ) == 3 && batch_kernels_cover((*sp)[0], (*sp)[1], (*sp)[2], img_ct);
     const bool own_short = covered && short_columns((*sp)[1]);
+    covered              = covered && ! (own_short && capturing);
     plan->plan_batched   = covered && ! own_short;
     if ( n > 0 )
-        rc = setup_subframe(plan, covered);
+        rc = setup_subframe(plan, covered, capturing);
     if ( ! rc && plan->sub_active )
         rc = setup_batch_kernels(plan, plan->sub_xc, CpxT::c64);
     if ( rc && plan->sub_small && forgive_no_memory(rc) ) { // no memory for a small frame: the batch does without
