@@ -220,16 +220,19 @@ static hipError_t go_full_wave(const Stage& s, const StageIO& io, const float2* 
 
 // Real rows of 1024 .. 8192 points into a transposed spectrum, two rows as one complex
 // line (pair_rows.hpp), PPW pairs per workgroup.
+template <int N, int PPW, typename TIn, bool PAD>
+static hipError_t go_pair_rows_t(const Stage& s, const StageIO& io, const float2* tw, hipStream_t st) {
+    const dim3 grid((unsigned)(((s.nlines + 1) / 2 + PPW - 1) / PPW)), block(N / kPairE * PPW);
+    launch_kernel<k_r2c_pair_rows<N, PPW, TIn, PAD>>(grid, block, 0, st, static_cast<const TIn*>(io.src), to_device(s.im), s.L,
+            static_cast<float2*>(io.dst), to_device(s.om), s.nout, s.nlines, io.scale, tw);
+    return hipGetLastError( );
+}
+
 template <int N, int PPW>
 static hipError_t go_pair_rows(const Stage& s, const StageIO& io, const float2* tw, hipStream_t st) {
-    const dim3 grid((unsigned)(((s.nlines + 1) / 2 + PPW - 1) / PPW)), block(N / kPairE * PPW);
     if ( io.src_rt == RealT::f32 )
-        launch_kernel<k_r2c_pair_rows<N, PPW, float>>(grid, block, 0, st, static_cast<const float*>(io.src), to_device(s.im),
-                s.L, static_cast<float2*>(io.dst), to_device(s.om), s.nout, s.nlines, io.scale, tw);
-    else
-        launch_kernel<k_r2c_pair_rows<N, PPW, __half>>(grid, block, 0, st, static_cast<const __half*>(io.src),
-                to_device(s.im), s.L, static_cast<float2*>(io.dst), to_device(s.om), s.nout, s.nlines, io.scale, tw);
-    return hipGetLastError( );
+        return s.L < s.N ? go_pair_rows_t<N, PPW, float, true>(s, io, tw, st) : go_pair_rows_t<N, PPW, float, false>(s, io, tw, st);
+    return s.L < s.N ? go_pair_rows_t<N, PPW, __half, true>(s, io, tw, st) : go_pair_rows_t<N, PPW, __half, false>(s, io, tw, st);
 }
 
 static hipError_t try_pair_rows(const Stage& s, const StageIO& io, const float2* tw, hipStream_t st) {

@@ -74,13 +74,13 @@ __device__ __forceinline__ int line_table_index(int g) {
 template <int N, int E, int NT>
 struct LineTable {
     static constexpr int SIZE = line_table_size<N, E>( ), ROWS = (SIZE + NT - 1) / NT;
-    float2               w[ROWS];
+    bits_t<float2>       w[ROWS];
     __device__ __forceinline__ void load(const float2* __restrict__ twm) {
 #pragma unroll
         for ( int r = 0; r < ROWS; r++ ) {
             const int g = threadIdx.x + NT * r;
             if ( g < SIZE )
-                w[r] = load_cpx(as_global(twm), line_table_index<N, E>(g));
+                w[r] = load_bits(as_global(twm) + line_table_index<N, E>(g));
         }
     }
     __device__ __forceinline__ void store(float2* tab) const {
@@ -88,7 +88,7 @@ struct LineTable {
         for ( int r = 0; r < ROWS; r++ ) {
             const int g = threadIdx.x + NT * r;
             if ( g < SIZE )
-                tab[g] = w[r];
+                tab[g] = bits_value(w[r]);
         }
     }
 };

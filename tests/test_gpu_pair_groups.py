@@ -18,8 +18,9 @@ TOL = 2e-6  # FP32 against FP64, as in the other pair-row tests
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 NY = 2048
 
-# rows of a forward (160 workgroups' worth of pairs keep a group): 161, 321 and 641 pairs
-FORWARD = [(n, rows, group) for n in (1024, 2048, 4096, 8192) for rows, group in ((321, 1), (641, 2), (1281, 4))]
+# rows of a forward, padded and whole (160 workgroups' worth of pairs keep a group): 161, 321 and 641 pairs
+FORWARD = [(n, rows, length, group) for n in (1024, 2048, 4096, 8192) for rows, group in ((321, 1), (641, 2), (1281, 4))
+           for length in (n - n // 5, n)]
 # rows and window of an inverse: 160 workgroups' worth for windows of over half a row, 100 below (rows of over 1024
 # points come as pairs from 160 pairs on)
 INVERSE = [(n, rows, n // 2 if half else n // 2 + 3, group) for n in (1024, 2048, 4096, 8192)
@@ -27,8 +28,7 @@ INVERSE = [(n, rows, n // 2 if half else n // 2 + 3, group) for n in (1024, 2048
            if rows > 199 or n == 1024]
 
 
-def _forward(n, rows):
-    length = n - n // 5
+def _forward(n, rows, length):
     ft = H.make_plan((length, rows, 1), (n, NY, 1), (n, NY, 1), (n, NY, 1))
     img = np.random.default_rng(n + rows).standard_normal((rows, length)).astype(np.float32)
     out = H.dev_poison(ft.ReturnFwdOutputMemorySize())
@@ -44,10 +44,10 @@ def _inverse(n, rows, window):
     return spec, H.real_window(H.to_host(out), window, rows)
 
 
-@pytest.mark.parametrize("n,rows,group", FORWARD)
-def test_forward_groups(n, rows, group):
-    H.log(f"pair groups forward {n}, {rows} rows")
-    img, got = _forward(n, rows)
+@pytest.mark.parametrize("n,rows,length,group", FORWARD)
+def test_forward_groups(n, rows, length, group):
+    H.log(f"pair groups forward {length} -> {n}, {rows} rows")
+    img, got = _forward(n, rows, length)
     want = O.fwd_2d(H.padded_real(img, img.shape[1]), img.shape[1], n, NY)
     assert O.rel_l2(got, want) < TOL
 
@@ -64,7 +64,7 @@ def test_groups_of_the_launch_rule():
     """The pairs per workgroup named above are those that run (8192-point rows: at most two)."""
     H.log("pair groups from the launch log")
     code = ("from tests import test_gpu_pair_groups as T\n"
-            "for n, rows, _ in T.FORWARD: T._forward(n, rows)\n"
+            "for n, rows, length, _ in T.FORWARD: T._forward(n, rows, length)\n"
             "for n, rows, window, _ in T.INVERSE: T._inverse(n, rows, window)\n")
     r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=110,
                        env=dict(os.environ, FASTFFT_LOG="1"))
