@@ -7,7 +7,8 @@
 // N = P*Q is split decimation-in-frequency style:
 //   y_q[m]      = sum_s x[s P + m] W_Q^{s q}          (radix-Q pass over the line in LDS)
 //   X[Q k' + q] = FFT_P( y_q[m] W_N^{m q} )[k']         (wave q, register Stockham)
-// The line is read with coalesced loads into LDS, zeros from L on: a padded line costs
+// The line is read with coalesced loads into LDS, zeros from L on (PAD: L < N; whole lines
+// load without a branch per value, 2048^2 forward y-pass 10.0 us, 10.5 with it): a padded line costs
 // the arithmetic of a whole one but reads L values only, and the stores of the N outputs
 // bound it.  The generic line kernel, which runs one P-point transform per output residue
 // (P >= L) in turn, took 17.3 us for 257 lines of 64 in 512 points and 79 us for 2049 of
@@ -21,7 +22,7 @@
 
 namespace fastfft_amd {
 
-template <int P, int Q, typename TIn, bool REAL, typename TOut>
+template <int P, int Q, typename TIn, bool REAL, typename TOut, bool PAD>
 __global__ void __launch_bounds__(64 * Q)
         k_fwd_full_wave(const TIn* __restrict__ in, LineMap im, int L, TOut* __restrict__ out, LineMap om, int nout, int nlines,
                         float pre_scale, const float2* __restrict__ tw) {
@@ -48,7 +49,7 @@ __global__ void __launch_bounds__(64 * Q)
         for ( int r = 0; r < N / NT; r++ ) {
             const int n = threadIdx.x + NT * r;
             z[r]        = make_float2(0.f, 0.f);
-            if ( n < L ) {
+            if ( ! PAD || n < L ) {
                 if constexpr ( REAL )
                     z[r].x = load_real(lp, n * im.es);
                 else

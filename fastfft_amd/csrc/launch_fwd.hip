@@ -197,10 +197,13 @@ static hipError_t try_r2c_wave(const Stage& s, const StageIO& io, const float2* 
 // line, P = 512 (256 for N = 256) and Q = N / P.
 template <int P, int Q, typename TIn, bool REAL, typename TOut>
 static hipError_t go_full_wave_t(const Stage& s, const StageIO& io, const float2* tw, hipStream_t st) {
-    launch_kernel<k_fwd_full_wave<P, Q, TIn, REAL, TOut>>(dim3((unsigned)s.nlines), dim3(64 * Q), 0, st,
-            static_cast<const TIn*>(io.src), to_device(s.im), s.L, static_cast<TOut*>(io.dst), to_device(s.om), s.nout,
-            s.nlines, io.scale, tw);
-    return hipGetLastError( );
+    auto go = [&](auto pad) {
+        launch_kernel<k_fwd_full_wave<P, Q, TIn, REAL, TOut, decltype(pad)::value>>(dim3((unsigned)s.nlines), dim3(64 * Q), 0, st,
+                static_cast<const TIn*>(io.src), to_device(s.im), s.L, static_cast<TOut*>(io.dst), to_device(s.om), s.nout,
+                s.nlines, io.scale, tw);
+        return hipGetLastError( );
+    };
+    return s.L < s.N ? go(std::true_type{ }) : go(std::false_type{ });
 }
 
 template <int P, int Q>
