@@ -69,9 +69,8 @@ inline int env_int(const char* name, int dflt) {
 }
 
 // Calls f(N, PPW) for the pair-row kernels (pair_rows.hpp): rows of N points, PPW pairs per
-// workgroup, at most FASTFFT_PAIR_GROUP; not supported below min_pairs pairs (rows of 1024 points
-// are taken from one pair on: 128 rows 10.0 us, 10.6 on the row kernels; inverse 10.4 and 12.6).
-// All figures here and at the callers are times of whole 2-D transforms.
+// workgroup, at most FASTFFT_PAIR_GROUP; not supported where pair_rows_pay (plan.hpp) says no.
+// All figures here are times of whole 2-D transforms.
 // Four pairs make 64-byte segments (workgroups of 1024 threads at N = 4096; 8192-point rows fit
 // two): 4096^2 forward 67 us with one pair, 55 with two or four; 2730 rows of 4096 points 65, 48
 // and 44.  The group is halved below `groups` workgroups' worth of pairs, which keeps CUs busy.
@@ -83,7 +82,7 @@ inline int env_int(const char* name, int dflt) {
 template <class F>
 hipError_t pair_rows_dispatch(int N, int nrows, int min_pairs, int groups, F&& f) {
     const int npairs = (nrows + 1) / 2, cap = env_int("FASTFFT_PAIR_GROUP", 4);
-    if ( npairs < env_int("FASTFFT_PAIR_MIN", N == 1024 ? 1 : min_pairs) )
+    if ( ! pair_rows_pay(N, nrows, min_pairs) )
         return hipErrorNotSupported;
     int       g      = N == 8192 ? 2 : 4;
     while ( g > 1 && (g > cap || npairs < groups * g) )

@@ -244,9 +244,7 @@ static hipError_t try_pair_rows(const Stage& s, const StageIO& io, const float2*
          s.om.es % 2 != 0 || s.om.es < s.nlines ||
          reinterpret_cast<std::uintptr_t>(io.dst) % 16 != 0 || env_int("FASTFFT_NO_PAIR_LINES", 0) )
         return hipErrorNotSupported;
-    // From 65 pairs on (rows of more than 1024 points): 128 full rows of 4096 points 11.3 us on the
-    // row kernels and 12.5 as pairs, 170 rows of 3071 points 14.2 and 13.3, 256 full rows of 2048 a tie.
-    return pair_rows_dispatch(s.N, s.nlines, 65, 160, [&](auto nc, auto gc) {
+    return pair_rows_dispatch(s.N, s.nlines, kPairMinForward, 160, [&](auto nc, auto gc) {
         return go_pair_rows<decltype(nc)::value, decltype(gc)::value>(s, io, tw, st);
     });
 }

@@ -498,10 +498,7 @@ static hipError_t try_c2r_pair_rows(const Stage& s, const StageIO& io, const flo
          s.om.n2 != 1 || s.om.es != 1 || reinterpret_cast<std::uintptr_t>(io.src) % 16 != 0 ||
          env_int("FASTFFT_NO_PAIR_LINES", 0) || env_int("FASTFFT_NO_FULL_LINES", 0) )
         return hipErrorNotSupported;
-    // From 160 pairs on (rows of more than 1024 points): 256 rows of 4096 points 13.2 us on the row
-    // kernels and 14.4 as pairs, of 2048 points 10.7 and 11.9; 412 rows cut to 489 of 2048 points
-    // 18.4 and 16.4, to 1001 of 4096 points 25.2 and 21.4.
-    return pair_rows_dispatch(s.N, s.nlines, 160, 2 * s.M > s.N ? 160 : 100, [&](auto nc, auto gc) {
+    return pair_rows_dispatch(s.N, s.nlines, kPairMinInverse, 2 * s.M > s.N ? 160 : 100, [&](auto nc, auto gc) {
         return go_c2r_pair_rows<decltype(nc)::value, decltype(gc)::value>(s, io, tw, st);
     });
 }

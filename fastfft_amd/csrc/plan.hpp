@@ -100,6 +100,14 @@ void stage_list_workspace(const std::vector<Stage>& st, size_t& ws_a, size_t& ws
 // Sub-transform size for a line of N with L nonzero inputs and M kept outputs.
 int pick_sub_size(int N, int L, int M);
 
+// The pair-row kernels take nrows rows of N points of a 2-D FwdFFT or InvFFT from this many pairs on
+// (from one at 1024 points; FASTFFT_PAIR_MIN overrides it).  Whole 2-D transforms, us on the row kernels and as pairs:
+// 128 full rows of 4096 points forward 11.3 and 12.5, 170 rows of 3071 points 14.2 and 13.3, 256 full rows of 2048 a
+// tie; 256 rows of 4096 points inverse 13.2 and 14.4, of 2048 points 10.7 and 11.9, 412 rows cut to 489 of 2048 points
+// 18.4 and 16.4, to 1001 of 4096 points 25.2 and 21.4; 128 rows of 1024 points 10.6 and 10.0, inverse 12.6 and 10.4.
+constexpr int kPairMinForward = 65, kPairMinInverse = 160;
+bool          pair_rows_pay(int N, int nrows, int min_pairs);
+
 std::string describe(const PlanState& p, const std::vector<Stage>& stages);
 
 constexpr int kMaxSize2D = 8192; // twiddle table / largest line transform

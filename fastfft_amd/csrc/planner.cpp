@@ -162,11 +162,21 @@ static long ws_ld(int n) {
     return n + pad;
 }
 
+bool pair_rows_pay(int N, int nrows, int min_pairs) {
+    const char* v    = std::getenv("FASTFFT_PAIR_MIN");
+    const int   least = v && v[0] ? std::atoi(v) : N == 1024 ? 1 : min_pairs;
+    return N >= 1024 && (nrows + 1) / 2 >= least;
+}
+
 // Leading dimension of a workspace array of columns (2-D FwdFFT and InvFFT: A[kx][y]) of n
-// values: a multiple of 8, so that the 64-byte segments that the x-passes move (eight
-// neighbouring rows of one kx) are aligned, and an odd row count has its partner's slot.
-static long ws_ld_columns(int n) {
-    return (ws_ld(n) + 7) / 8 * 8;
+// values, the rows of an x-pass of N points: a multiple of 8 where the x-pass moves 64-byte
+// segments (eight neighbouring rows of one kx), so that those are aligned and an odd row count has
+// its partner's slot.  The row kernels of longer rows gather one row at a time: they keep n, as a
+// multiple of 8 is a power of two too often, which puts a row's values on few memory channels
+// (8192 x 1024 cut to 2045 x 251: C2R rows 14.3 us on columns of 251 values, 16.5 on 256).
+static long ws_ld_columns(int n, int N, int min_pairs) {
+    const long ld = ws_ld(n);
+    return N > 1024 && ! pair_rows_pay(N, n, min_pairs) ? ld : (ld + 7) / 8 * 8;
 }
 
 // Leading dimension of a row-major workspace array of n complex values per row:
@@ -218,7 +228,7 @@ static PlanError fwd_stages_2d(const PlanState& p, std::vector<Stage>& st, Buf f
     s1.im       = lm(pitch, 0, 1, 1);
     s1.dst      = Buf::ws_a;
     s1.dst_elem = Elem::cpx_f32;
-    s1.om       = lm(1, 0, ws_ld_columns(in.y), 1);
+    s1.om       = lm(1, 0, ws_ld_columns(in.y, Nx, kPairMinForward), 1);
     st.push_back(s1);
     // y-pass: each of the out.w columns A[kx][0..in.y) -> C[kx][ky]
     const int Ny = std::max(in.y, out.y);
@@ -227,7 +237,7 @@ static PlanError fwd_stages_2d(const PlanState& p, std::vector<Stage>& st, Buf f
                               Ny, in.y, 0, 0, out.y, out.w);
     s2.src      = Buf::ws_a;
     s2.src_elem = Elem::cpx_f32;
-    s2.im       = lm(ws_ld_columns(in.y), 0, 1, 1);
+    s2.im       = lm(ws_ld_columns(in.y, Nx, kPairMinForward), 0, 1, 1);
     s2.dst      = final_dst;
     s2.dst_elem = Elem::cpx_input_type;
     s2.om       = lm(out.y, 0, 1, 1);
@@ -295,14 +305,14 @@ static PlanError inv_stages_2d(const PlanState& p, std::vector<Stage>& st, Buf s
     s1.im       = lm(in.y, 0, 1, 1);
     s1.dst      = Buf::ws_b;
     s1.dst_elem = Elem::cpx_f32;
-    s1.om       = lm(ws_ld_columns(out.y), 0, 1, 1);
+    s1.om       = lm(ws_ld_columns(out.y, in.x, kPairMinInverse), 0, 1, 1);
     st.push_back(s1);
     // x-pass C2R on the out.y rows -> out[j][pitch]
     Stage s2    = make_stage(StageKind::inv_c2r, dec ? "c2r_decrease_XY" : "c2r_none_XY", in.x, 0, out.x,
                              axis_origin(p, 0, in.x, out.x), 0, out.y);
     s2.src      = Buf::ws_b;
     s2.src_elem = Elem::cpx_f32;
-    s2.im       = lm(1, 0, ws_ld_columns(out.y), 1);
+    s2.im       = lm(1, 0, ws_ld_columns(out.y, in.x, kPairMinInverse), 1);
     s2.dst      = Buf::user_out;
     s2.dst_elem = Elem::real_input_type;
     s2.om       = lm(2 * out.w, 0, 1, 1);
