@@ -27,16 +27,16 @@
 
 namespace fastfft_amd {
 
-// Values per thread: 16 at 128 points; 8 at 64 (twice the threads of short lines), at 512 (16 needs a radix-2 pass after the same two
-// exchanges: 512-point passes of 512^3 143 + 48 us against 118 + 42) and at 256 points, where
-// twice the waves outweigh the second exchange (fused z-pass of 256^3 35.3 us with 16, 30.4
-// with 8; C2R rows 9.6 and 8.6) except for real rows (6.9 and 8.7 us for 5,084 of them).
-constexpr int line_values(int N, bool real_in) { return N == 64 || N == 512 || (N == 256 && ! real_in) ? 8 : 16; }
+// Values per thread: 8, and 16 for real rows of 256 points (5,084 of them 6.9 us with 16, 8.7 with 8).
+// Twice the threads of a line outweigh the exchange that 16 values save at 64, 128 and 256 points (128^2
+// forward 8.2 us with 16, 6.6 with 8, inverse 9.2 and 7.0; fused z-pass of 256^3 35.3 and 30.4, its C2R rows 9.6
+// and 8.6), and at 512 points 16 values need as many exchanges (512^3 cut to 128^3: 143 + 48 us and 118 + 42).
+constexpr int line_values(int N, bool real_in) { return N == 256 && real_in ? 16 : 8; }
 template <typename T>
 constexpr bool is_real_element = std::is_same<T, float>::value || std::is_same<T, __half>::value;
 constexpr int kTileLines = 16; // transforms of a workgroup whose lanes run across lines
 
-// LDS slot of element k of a line: one pad slot per 16, and 2 more per line, so that the
+// LDS slot of element k of a line: one pad slot per E values, and 2 more per line, so that the
 // scatters and gathers of both arrangements are free of bank conflicts but for single lanes.
 template <int E>
 __device__ __forceinline__ int line_slot(int k) {
