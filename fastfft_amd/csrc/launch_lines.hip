@@ -49,8 +49,22 @@ static bool line_groups(const Stage& s, const HostLineMap& m) {
            (long)s.N * m.es + 256 * step < (1L << 28);
 }
 
+// Few 256-point lines of a 2-D pass: the kernels of one wave per line (k_fwd_full_wave, k_inv_full_wave,
+// k_inv_window_rows) fill more of the chip.  2-D transforms, us here and there: 256^2 forward 7.5 and 6.7, inverse 7.6
+// and 6.9, cut to 61 x 59 7.1 and 6.4; 256 rows of 64 values in 256 x 1024 8.5 and 8.0.  Rows: a tie at 512 (256 x 512
+// forward 7.9 and 7.9), behind at 682 (8.8 and 9.4, 191 values each in 256 x 1024).  Unit-stride complex lines, inverse:
+// 513 of 1024 x 256 cut to 253 x 59 8.9 and 8.5, 1025 of 2048 x 256 9.8 and 9.6, 2049 of 4096 x 256 11.9 and 12.0;
+// forward: 513 of 1024 x 256 8.5 and 9.0.
+static bool few_lines(const Stage& s) {
+    if ( s.N != 256 || s.im.n2 != 1 || s.om.n2 != 1 )
+        return false;
+    return s.kind == StageKind::inv_c2r || s.kind == StageKind::fwd_real ? s.nlines <= 256
+                                                                         : s.im.es == 1 && s.om.es == 1 &&
+                                                                                   s.nlines <= (s.kind == StageKind::fwd_cpx ? 300 : 1100);
+}
+
 bool lines_cover(const Stage& s) {
-    if ( ! (s.N == 64 || s.N == 128 || s.N == 256 || s.N == 512) || s.nlines <= 0 || ! line_groups(s, s.im) ||
+    if ( ! (s.N == 64 || s.N == 128 || s.N == 256 || s.N == 512) || s.nlines <= 0 || few_lines(s) || ! line_groups(s, s.im) ||
          ! line_groups(s, s.om) )
         return false;
     if ( s.kind == StageKind::inv_c2r )
