@@ -7,9 +7,9 @@
 //   X[Q k' + q] = FFT_P( W_N^{m q} sum_s a[s P + m] W_Q^{s q} )[k'],   m < P, s P + m < L
 //   U_q         = IFFT_P( img[Q k' + q] conj(X[Q k' + q]) )
 // and leaves U_q in LDS; each output takes y[o + j] = sum_q W_N^{-(o + j) q} U_q[(o + j) mod P]
-// by Horner's rule in W_N^{-(o + j)}, one table entry: no product per value of the sub-
-// transforms, and nothing of the window in their registers.  (Windows of over a quarter of the
-// column take one radix-Q pass instead, which costs less than Horner's rule there.)  The image values are loaded
+// in log2 Q steps (share_sum): no product per value of the sub-transforms, and nothing of the
+// window in their registers.  (Windows of over a quarter of the column take one radix-Q pass
+// instead, which costs less there.)  The image values are loaded
 // before the template's transform and the Stockham twiddles are read from LDS at their use,
 // which leaves 76 registers, three workgroups of
 // 8 waves per CU.  Bound by VALU issue: 4096^2 with a 384^2 template and a 512^2 window takes
@@ -66,6 +66,17 @@ __device__ __forceinline__ void wave_passes(float2 (&v)[P / 64], float2* __restr
     }
 }
 
+// sum_q W^q u[q PITCH], q < Q, with w[l] = conj W^{2^l}: the two halves' sums and one product, log2 Q
+// products deep.  (Horner's rule in W, Q - 1 deep, puts a rounding of the whole sum at each step: rel-L2 error
+// against 64 bits of small windows of 2048 x 8192 3.3e-7, here 2.6e-7; of 4096^2 2.8e-7 and 2.6e-7, 42.4 us both.)
+template <int Q, int PITCH, int LQ>
+__device__ __forceinline__ float2 share_sum(const float2* u, const float2 (&w)[LQ]) {
+    if constexpr ( Q == 1 )
+        return u[0];
+    else
+        return cadd(share_sum<Q / 2, PITCH>(u, w), cmulc(share_sum<Q / 2, PITCH>(u + Q / 2 * PITCH, w), w[__builtin_ctz(Q / 2)]));
+}
+
 // Grid: nlines - 1 workgroups when pack_ends (columns 0 and last_line share workgroup 0), else
 // nlines.  Element n of template column c is a[c lda + n a_es], of image column c img[c ldg + n],
 // output j out[c ldo + j o_es]; 0 <= o < N.
@@ -74,7 +85,7 @@ __global__ void __launch_bounds__(64 * Q) __attribute__((amdgpu_waves_per_eu(6))
         k_xcorr_one(const float2* __restrict__ a, long lda, long a_es, int L, const TImg* __restrict__ img, long ldg,
                     float2* __restrict__ out, long ldo, long o_es, int M, int o, float scale, const float2* __restrict__ tw,
                     int last_line, int pack_ends) {
-    constexpr int T = 64, E = P / T, N = P * Q, NT = T * Q;
+    constexpr int T = 64, E = P / T, N = P * Q, NT = T * Q, LQ = Q > 1 ? __builtin_ctz(Q) : 1;
     using FFT       = WaveFFT<P>;
     static_assert(FFT::SLOTS == P, "the workgroup's regions hold a whole column");
     __shared__ float2 lds[Q * P];
@@ -196,13 +207,12 @@ __global__ void __launch_bounds__(64 * Q) __attribute__((amdgpu_waves_per_eu(6))
             wl[t + T * i] = v[i];
         __syncthreads( );
         for ( int j = threadIdx.x; j < M; j += NT ) {
-            const int    x   = (o + j) & (N - 1), m = x & (P - 1);
-            const float2 w   = load_cpx(as_global(twm) + N, x); // W_N^{o + j}
-            float2       acc = lds[(Q - 1) * P + m];
+            const int x = (o + j) & (N - 1);
+            float2    w[LQ];
 #pragma unroll
-            for ( int qq = Q - 2; qq >= 0; qq-- )
-                acc = cadd(cmulc(acc, w), lds[qq * P + m]);
-            store(j, acc);
+            for ( int l = 0; l < LQ; l++ ) // W_N^{x 2^l} = W_{N / 2^l}^x
+                w[l] = load_cpx(as_global(twm) + (N >> l), x & ((N >> l) - 1));
+            store(j, share_sum<Q, P>(lds + (x & (P - 1)), w));
         }
     };
     if ( ends )
