@@ -87,8 +87,8 @@ static hipError_t try_xcorr_col(const Stage& s, const StageIO& io, const float2*
     }
 }
 
-// One template, any length, window and origin: one workgroup per column of 256 to 8192 points
-// with P = 512 (256 for N = 256), columns 0 and nlines - 1 in one workgroup as above.
+// One template, any length, window and origin: one workgroup per column of 256 to 8192 points,
+// columns 0 and nlines - 1 in one workgroup as above.
 template <int P, int Q, typename TImg>
 static hipError_t go_xcorr_one(const Stage& s, const StageIO& io, const float2* tw, hipStream_t st) {
     const int pack = s.real_end_lines && s.nlines >= 2 && env_int("FASTFFT_XCORR_PACK", 1) ? 1 : 0;
@@ -100,13 +100,17 @@ static hipError_t go_xcorr_one(const Stage& s, const StageIO& io, const float2* 
 
 template <typename TImg>
 static hipError_t try_xcorr_one(const Stage& s, const StageIO& io, const float2* tw, hipStream_t st) {
+    // Sub-transforms of 512 points, but of 256 for short columns, whose few waves leave the chip idle
+    // (512^2 with 64^2 and 256^2 15.2 us with 512, 13.9 with 256; 1024^2 with 256^2 and 256^2 18.5 and 17.0; 4096 x 512
+    // with 1/16 and 1/8 of each axis 14.3 and 13.9; a tie at 2048 points), and of 1024 for 8192, where 16 waves of 512 leave
+    // one workgroup per CU (8192^2 with 512^2 and 1024^2 220 and 177; 4096^2 40.8 us with 512, 45.9 with 1024).
     switch ( s.N ) {
         case 256: return go_xcorr_one<256, 1, TImg>(s, io, tw, st);
-        case 512: return go_xcorr_one<512, 1, TImg>(s, io, tw, st);
-        case 1024: return go_xcorr_one<512, 2, TImg>(s, io, tw, st);
+        case 512: return go_xcorr_one<256, 2, TImg>(s, io, tw, st);
+        case 1024: return go_xcorr_one<256, 4, TImg>(s, io, tw, st);
         case 2048: return go_xcorr_one<512, 4, TImg>(s, io, tw, st);
         case 4096: return go_xcorr_one<512, 8, TImg>(s, io, tw, st);
-        case 8192: return go_xcorr_one<512, 16, TImg>(s, io, tw, st);
+        case 8192: return go_xcorr_one<1024, 8, TImg>(s, io, tw, st);
         default: return hipErrorNotSupported;
     }
 }

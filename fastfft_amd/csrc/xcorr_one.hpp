@@ -81,7 +81,7 @@ __device__ __forceinline__ float2 share_sum(const float2* u, const float2 (&w)[L
 // nlines.  Element n of template column c is a[c lda + n a_es], of image column c img[c ldg + n],
 // output j out[c ldo + j o_es]; 0 <= o < N.
 template <int P, int Q, typename TImg>
-__global__ void __launch_bounds__(64 * Q) __attribute__((amdgpu_waves_per_eu(6)))
+__global__ void __launch_bounds__(64 * Q) __attribute__((amdgpu_waves_per_eu(P == 1024 ? 4 : 6)))
         k_xcorr_one(const float2* __restrict__ a, long lda, long a_es, int L, const TImg* __restrict__ img, long ldg,
                     float2* __restrict__ out, long ldo, long o_es, int M, int o, float scale, const float2* __restrict__ tw,
                     int last_line, int pack_ends) {
