@@ -712,9 +712,11 @@ static fastfft_status setup_batch_kernels(fastfft_plan p, const std::vector<Stag
             best.p = 0;
     }
     else if ( p->sub_active && (p->sub_raised || p->sub_fy < 512) && ! env_flag("FASTFFT_TUNE") ) {
-        // small frames: no timing at set-up; launches of the whole batch, up to 64 templates, a few
-        // templates per group of columns (24 templates of at most 78^2 in 2048 x 1024: 55 us, 41 of
-        // at most 53^2 in 1024 x 512: 53 us)
+        // raised and short frames: no timing at set-up; launches of the whole batch, up to 64 templates, a few
+        // templates per group of columns.  4 to 100 templates on frames of 512 x 256 to 2048 x 2048, which these
+        // kernels end at (64 templates: at most 0.8 GB of slots), take at most 8 % more than the shape that timing
+        // finds (100 templates of 1000 x 500 on 2048 x 1024 1088 us, 1041; on 2048 x 2048 1950, 1946), and where
+        // timing's powers of two leave a second launch, less (24 of at most 400^2 on 1024 x 1024 103 us, 124)
         best.chunk = std::min(n, 64);
         best.group = n >= 32 ? 4 : n >= 8 ? 2 : 1;
         how        = "default";
@@ -989,8 +991,11 @@ static fastfft_status setup_frame(fastfft_plan p, int fx, int fy, bool capturing
 // quarter of the plan's.  Where the batched kernels take neither that frame nor the plan's own
 // stages, a batch of four templates or more goes to a frame of at least 512 x 256 points, the
 // shortest those kernels take, up to the plan's size: the alternative is three launches or more
-// per template (24 templates of at most 78^2 in 2048 x 1024: 419 us).  FASTFFT_NO_SUBFRAME
-// leaves both off.
+// per template.  Four templates, us per template and on the frame: 51 x 25 in 1024 x 512 72 and 36,
+// 400^2 in 1024^2 78 and 56 (a frame of 1024^2), 1000 x 500 in 2048 x 1024 107 and 94 (2048 x 1024), 1000^2 in
+// 4096 x 2048 180 and 156 (2048^2).  In 2048^2 the reduction to a frame of 2048^2 costs more than it
+// saves four templates (1000^2 129 and 145, 600^2 117 and 126; five 162 and 160, 145 and 141).
+// FASTFFT_NO_SUBFRAME leaves both off.
 static fastfft_status setup_subframe(fastfft_plan p, bool plan_covered, bool capturing) {
     free_subframe(p);
     if ( env_flag("FASTFFT_NO_SUBFRAME") || p->st.transform_dimension != 2 )
@@ -1000,10 +1005,12 @@ static fastfft_status setup_subframe(fastfft_plan p, bool plan_covered, bool cap
     if ( fx < nn.x && fy < nn.y && 4L * fx * fy <= (long)nn.x * nn.y )
         if ( auto rc = setup_frame(p, fx, fy, capturing); rc || p->sub_active )
             return rc;
-    if ( plan_covered || capturing || p->batch.size( ) < 4 || nn.x < 512 || nn.y < 256 )
+    if ( plan_covered || capturing || nn.x < 512 || nn.y < 256 )
         return ok( );
-    if ( auto rc = setup_frame(p, std::min(std::max(fx, 512), nn.x), std::min(std::max(fy, 256), nn.y), capturing);
-         rc && ! forgive_no_memory(rc) )
+    const int rx = std::min(std::max(fx, 512), nn.x), ry = std::min(std::max(fy, 256), nn.y);
+    if ( p->batch.size( ) < (rx == nn.x && ry == nn.y && (long)rx * ry >= 2048L * 2048 ? 5 : 4) )
+        return ok( );
+    if ( auto rc = setup_frame(p, rx, ry, capturing); rc && ! forgive_no_memory(rc) )
         return rc;
     p->sub_raised = p->sub_small = p->sub_active;
     return ok( );

@@ -45,3 +45,10 @@ def test_answers_of_short_columns(n, size, window, origin, count, frame, answers
                                                      ((300, 100), (200, 100), 1, "full"), ((300, 100), (200, 100), 2, "512x256")])
 def test_one_template_runs_on_the_plans_stages(size, window, count, frame):
     assert _batch((2048, 2048), size, window, (-100, -50), count)[1]["frame"] == frame
+
+
+@pytest.mark.parametrize("n,count,frame", [((2048, 2048), 4, "full"), ((2048, 2048), 5, "2048x2048"), ((4096, 2048), 4, "2048x2048"),
+                                           ((4096, 2048), 3, "full")])
+def test_four_templates_do_not_pay_for_a_whole_plan_frame(n, count, frame):
+    """Templates of 1000^2 whose lags need 2048 x 2048 points: the frame is the plan's own size, or half of it."""
+    assert _batch(n, (1000, 1000), (1000, 500), (-500, -250), count)[1]["frame"] == frame
