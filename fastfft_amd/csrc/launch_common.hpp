@@ -78,13 +78,15 @@ inline int env_int(const char* name, int dflt) {
 // 4096 points 17.7, 18.0 and 21.1 us forward with one, two and four pairs, 17.5, 19.1 and 23.1
 // inverse; 682 rows 25.5, 23.2 and 25.6 forward; 1365 rows 39.0, 31.5 and 29.3.  100 for smaller
 // windows, whose 64-byte reads count for more: 924 rows of 1024 points 18.6, 16.2 and 14.9 us, of
-// 2048 points 26.2, 22.7 and 20.8; 384 rows of 8192 points 25.5 with one pair, 30.4 with two.
+// 2048 points 26.2, 22.7 and 20.8.  8192-point rows keep single pairs up to 512 of them, which
+// are all in flight at once, two to a CU: 1024 rows forward 38.7 us with one, 39.1 with two,
+// inverse 34.7 and 37.0, 512 rows cut to 3001 values 25.0 and 32.1; 1300 rows 67.7 and 57.5, 79.0 and 61.1.
 template <class F>
 hipError_t pair_rows_dispatch(int N, int nrows, int min_pairs, int groups, F&& f) {
     const int npairs = (nrows + 1) / 2, cap = env_int("FASTFFT_PAIR_GROUP", 4);
     if ( ! pair_rows_pay(N, nrows, min_pairs) )
         return hipErrorNotSupported;
-    int       g      = N == 8192 ? 2 : 4;
+    int       g      = N < 8192 ? 4 : npairs > 512 ? 2 : 1;
     while ( g > 1 && (g > cap || npairs < groups * g) )
         g /= 2;
     auto by_n = [&](auto nc) -> hipError_t {

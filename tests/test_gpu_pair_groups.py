@@ -61,7 +61,7 @@ def test_inverse_groups(n, rows, window, group):
 
 
 def test_groups_of_the_launch_rule():
-    """The pairs per workgroup named above are those that run (8192-point rows: at most two)."""
+    """The pairs per workgroup named above are those that run (8192-point rows: two above 512 pairs, else one)."""
     H.log("pair groups from the launch log")
     code = ("from tests import test_gpu_pair_groups as T\n"
             "for n, rows, length, _ in T.FORWARD: T._forward(n, rows, length)\n"
@@ -70,4 +70,4 @@ def test_groups_of_the_launch_rule():
                        env=dict(os.environ, FASTFFT_LOG="1"))
     assert r.returncode == 0, r.stderr[-2000:]
     got = [(int(n), int(g)) for n, g in re.findall(r"launch k_(?:r2c|c2r)_pair_rows<(\d+), (\d+),", r.stderr)]
-    assert got == [(c[0], min(c[-1], 2 if c[0] == 8192 else 4)) for c in FORWARD + INVERSE]
+    assert got == [(n, group if n < 8192 else 2 if rows > 1024 else 1) for n, rows, _, group in FORWARD + INVERSE]
