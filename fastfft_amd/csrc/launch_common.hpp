@@ -70,24 +70,21 @@ inline int env_int(const char* name, int dflt) {
 
 // Calls f(N, PPW) for the pair-row kernels (pair_rows.hpp): rows of N points, PPW pairs per
 // workgroup, at most FASTFFT_PAIR_GROUP; not supported where pair_rows_pay (plan.hpp) says no.
-// All figures here are times of whole 2-D transforms.
 // Four pairs make 64-byte segments (workgroups of 1024 threads at N = 4096; 8192-point rows fit
-// two): 4096^2 forward 67 us with one pair, 55 with two or four; 2730 rows of 4096 points 65, 48
-// and 44.  The group is halved below `groups` workgroups' worth of pairs, which keeps CUs busy.
-// 160, where the rows outweigh the segments (forward, and windows of over half a row): 512 rows of
-// 4096 points 17.7, 18.0 and 21.1 us forward with one, two and four pairs, 17.5, 19.1 and 23.1
-// inverse; 682 rows 25.5, 23.2 and 25.6 forward; 1365 rows 39.0, 31.5 and 29.3.  100 for smaller
-// windows, whose 64-byte reads count for more: 924 rows of 1024 points 18.6, 16.2 and 14.9 us, of
-// 2048 points 26.2, 22.7 and 20.8.  8192-point rows keep single pairs up to 512 of them, which
-// are all in flight at once, two to a CU: 1024 rows forward 38.7 us with one, 39.1 with two,
-// inverse 34.7 and 37.0, 512 rows cut to 3001 values 25.0 and 32.1; 1300 rows 67.7 and 57.5, 79.0 and 61.1.
+// two).  The group is halved below 160 workgroups' worth of pairs, which keeps CUs busy.  Whole 2-D
+// transforms, us with one, two and four pairs: 509 whole rows of 4096 points forward 15.8, 16.0 and
+// 19.8, inverse 16.1, 17.6 and 22.2; 809 rows 24.1, 21.8, 25.6 and 23.6, 22.5, 27.1; 1281 rows 29.5, 29.6,
+// 29.3 and 27.4, 26.5, 28.7; 4091 rows 66.1, 62.1, 53.4 and 61.9, 58.1, 57.9; 1281 rows of 2048 points cut to
+// 509 values 19.8, 18.9 and 18.2.  8192-point rows keep single pairs up to 512 of them, which are all in
+// flight at once, two to a CU: 509 rows inverse 27.4 with one and 33.5 with two, 1024 rows forward 38.4 and
+// 38.8, inverse 34.4 and 37.1; 2045 rows 64.4 and 60.0, 60.4 and 59.4.
 template <class F>
-hipError_t pair_rows_dispatch(int N, int nrows, int min_pairs, int groups, F&& f) {
+hipError_t pair_rows_dispatch(int N, int nrows, int min_pairs, F&& f) {
     const int npairs = (nrows + 1) / 2, cap = env_int("FASTFFT_PAIR_GROUP", 4);
     if ( ! pair_rows_pay(N, nrows, min_pairs) )
         return hipErrorNotSupported;
     int       g      = N < 8192 ? 4 : npairs > 512 ? 2 : 1;
-    while ( g > 1 && (g > cap || npairs < groups * g) )
+    while ( g > 1 && (g > cap || (N < 8192 && npairs < 160 * g)) )
         g /= 2;
     auto by_n = [&](auto nc) -> hipError_t {
         constexpr int NN = decltype(nc)::value;

@@ -244,7 +244,7 @@ static hipError_t try_pair_rows(const Stage& s, const StageIO& io, const float2*
          s.om.es % 2 != 0 || s.om.es < s.nlines ||
          reinterpret_cast<std::uintptr_t>(io.dst) % 16 != 0 || env_int("FASTFFT_NO_PAIR_LINES", 0) )
         return hipErrorNotSupported;
-    return pair_rows_dispatch(s.N, s.nlines, kPairMinForward, 160, [&](auto nc, auto gc) {
+    return pair_rows_dispatch(s.N, s.nlines, kPairMinForward, [&](auto nc, auto gc) {
         return go_pair_rows<decltype(nc)::value, decltype(gc)::value>(s, io, tw, st);
     });
 }

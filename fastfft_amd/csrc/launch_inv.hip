@@ -498,7 +498,7 @@ static hipError_t try_c2r_pair_rows(const Stage& s, const StageIO& io, const flo
          s.om.n2 != 1 || s.om.es != 1 || reinterpret_cast<std::uintptr_t>(io.src) % 16 != 0 ||
          env_int("FASTFFT_NO_PAIR_LINES", 0) || env_int("FASTFFT_NO_FULL_LINES", 0) )
         return hipErrorNotSupported;
-    return pair_rows_dispatch(s.N, s.nlines, kPairMinInverse, 2 * s.M > s.N ? 160 : 100, [&](auto nc, auto gc) {
+    return pair_rows_dispatch(s.N, s.nlines, kPairMinInverse, [&](auto nc, auto gc) {
         return go_c2r_pair_rows<decltype(nc)::value, decltype(gc)::value>(s, io, tw, st);
     });
 }

@@ -40,6 +40,15 @@ __device__ __forceinline__ int xcd_row(int b, int nrows) {
     return (b % kXcds) * (nrows / kXcds) + b / kXcds;
 }
 
+// The same for any count: XCD x takes ceil or floor of n / 8 consecutive indexes, the longer ranges
+// first.  Where workgroups share cache lines (the transposed side of the pair rows), the identity makes
+// every XCD read or write all of them: 509 rows of 8192 points inverse 38.5 us, 27.4 here, of 4096 points
+// forward 18.1 and 15.8.
+__device__ __forceinline__ int xcd_range(int b, int n) {
+    const int x = b % kXcds;
+    return x * (n / kXcds) + min(x, n % kXcds) + b / kXcds;
+}
+
 // Descriptor i of a batched launch (i wave-uniform), by scalar loads.
 __device__ __forceinline__ RowBatchItem load_item(const RowBatchItem* items, int i) {
     const auto*  p = as_const(items + i);

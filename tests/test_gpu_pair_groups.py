@@ -21,10 +21,10 @@ NY = 2048
 # rows of a forward, padded and whole (160 workgroups' worth of pairs keep a group): 161, 321 and 641 pairs
 FORWARD = [(n, rows, length, group) for n in (1024, 2048, 4096, 8192) for rows, group in ((321, 1), (641, 2), (1281, 4))
            for length in (n - n // 5, n)]
-# rows and window of an inverse: 160 workgroups' worth for windows of over half a row, 100 below (rows of over 1024
-# points come as pairs from 160 pairs on)
+# rows and window of an inverse, windows of over half a row and of less (rows of over 1024 points come as pairs from 160
+# pairs on)
 INVERSE = [(n, rows, n // 2 if half else n // 2 + 3, group) for n in (1024, 2048, 4096, 8192)
-           for rows, half, group in ((321, False, 1), (641, False, 2), (1281, False, 4), (199, True, 1), (401, True, 2), (801, True, 4))
+           for rows, half, group in ((321, False, 1), (641, False, 2), (1281, False, 4), (199, True, 1), (401, True, 1), (801, True, 2))
            if rows > 199 or n == 1024]
 
 
