@@ -11,10 +11,11 @@
 // window in their registers.  (Windows of over a quarter of the column take one radix-Q pass
 // instead, which costs less there.)  The image values are loaded
 // before the template's transform and the Stockham twiddles are read from LDS at their use,
-// which leaves 76 registers, three workgroups of
-// 8 waves per CU.  Bound by VALU issue: 4096^2 with a 384^2 template and a 512^2 window takes
-// 29.9 us (82 MB), where the form with a product per value and 128 registers took 33.6; capped
-// at 64 registers 11 spill (39.5 us).
+// which leaves 76 registers, three workgroups of 8 waves per CU.  No unit is saturated: 4096^2 with
+// a 384^2 template and a 512^2 window (82 MB) keeps the VALU busy 65 % of its 30.9 us, the address
+// units 60 % (the waves' image values share their lines) and the LDS 34 %, and waves wait for
+// data and for their turn alike; the form with a product per value and 128 registers took 33.6 us.
+// Capped at 64 registers 11 spill (39.5 us).
 //
 // DC and Nyquist columns (0 and last_line of a real transform): workgroup 0 takes both as one
 // complex column, as described in xcorr_col.hpp.
@@ -68,7 +69,8 @@ __device__ __forceinline__ void wave_passes(float2 (&v)[P / 64], float2* __restr
 
 // sum_q W^q u[q PITCH], q < Q, with w[l] = conj W^{2^l}: the two halves' sums and one product, log2 Q
 // products deep.  (Horner's rule in W, Q - 1 deep, puts a rounding of the whole sum at each step: rel-L2 error
-// against 64 bits of small windows of 2048 x 8192 3.3e-7, here 2.6e-7; of 4096^2 2.8e-7 and 2.6e-7, 42.4 us both.)
+// against 64 bits of small windows of 4096^2 2.8e-7, here 2.65e-7; of 1024 x 8192 with sixteen shares 3.1e-7, with
+// eight 2.8e-7, here 2.65e-7.)
 template <int Q, int PITCH, int LQ>
 __device__ __forceinline__ float2 share_sum(const float2* u, const float2 (&w)[LQ]) {
     if constexpr ( Q == 1 )
@@ -209,9 +211,15 @@ __global__ void __launch_bounds__(64 * Q) __attribute__((amdgpu_waves_per_eu(P =
         for ( int j = threadIdx.x; j < M; j += NT ) {
             const int x = (o + j) & (N - 1);
             float2    w[LQ];
+            // W_N^{x 2^l}: two entries W_{N / 2^l}^x of the table, then squares (all from the table, 1 % more accurate, takes
+            // 2 % more of 4096^2 with 1021^2 and 1019^2: the loads' addresses)
 #pragma unroll
-            for ( int l = 0; l < LQ; l++ ) // W_N^{x 2^l} = W_{N / 2^l}^x
-                w[l] = load_cpx(as_global(twm) + (N >> l), x & ((N >> l) - 1));
+            for ( int l = 0; l < LQ; l++ ) {
+                if ( l < 2 )
+                    w[l] = load_cpx(as_global(twm) + (N >> l), x & ((N >> l) - 1));
+                else
+                    w[l] = make_float2(fmaf(w[l - 1].x, w[l - 1].x, -w[l - 1].y * w[l - 1].y), 2.f * w[l - 1].x * w[l - 1].y);
+            }
             store(j, share_sum<Q, P>(lds + (x & (P - 1)), w));
         }
     };
