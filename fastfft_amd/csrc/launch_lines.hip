@@ -20,10 +20,10 @@ static hipError_t go_lines_t(const Stage& s, const StageIO& io, const float2* tw
 }
 
 // Lines per workgroup: 16 (tiles), or 256 threads' worth of unit-stride lines, where that leaves at
-// least FASTFFT_LINES_MIN workgroups, else a quarter.  128 workgroups, half the CUs: 64^2 padded to
-// 512^2 and back takes 21.7 us with the large workgroups alone, 18.8 with the small ones, 64^3
-// forward 13.9 and 15.2, 64^3 padded to 256^3 34.9 and 39.6, 512^3 cut to 128^3 214 and 269; the
-// rule takes 19.1, 12.4, 34.4 and 209.
+// least FASTFFT_LINES_MIN workgroups, else a quarter.  128 workgroups, half the CUs.  Transforms in a
+// graph, us with the large workgroups alone, with the small ones and by the rule: 64^2 padded to 512^2 8.1, 6.8
+// and 6.8, 512^2 inverse 10.2, 8.2 and 8.1, 64^3 forward 9.4, 9.9 and 9.0, 64^3 padded to 256^3 31.6, 36.8 and
+// 31.7, 512^3 cut to 128^3 171, 235 and 171.
 template <int N, int DIR, typename TIn, bool HERM, typename TOut, bool IX, bool OX>
 static hipError_t go_lines(const Stage& s, const StageIO& io, const float2* tw, hipStream_t st, int M, int o) {
     constexpr int ROWS = HERM ? 2 : 1, BIG = IX || OX ? kTileLines : 256 * line_values(N, is_real_element<TIn>) / N, SMALL = BIG / 4;
